@@ -467,10 +467,10 @@ int prefill_chunk(const plh_model* m, const int* tokens, int T, int pos0, const 
   for (int l = 0; l < m->n_layers; ++l) {
     const plh_layer& L = m->layers[l];
     // model.c:988-1017: rmsnorm, q / k / v projections, biases where present
-    if (launch_rmsnorm_rows(a.x, L.attn_norm, a.xn, E, T, eps) ||
-        gemv_launch(call(L.q, E, Q, a.xn, E, a.q, Q, L.q_bias, nullptr, nullptr)) ||
-        gemv_launch(call(L.k, E, KV, a.xn, E, a.k, KV, L.k_bias, nullptr, nullptr)) ||
-        gemv_launch(call(L.v, E, KV, a.xn, E, a.v, KV, L.v_bias, nullptr, nullptr)))
+    const GemvCall qkv[3] = {call(L.q, E, Q, a.xn, E, a.q, Q, L.q_bias, nullptr, nullptr),
+                             call(L.k, E, KV, a.xn, E, a.k, KV, L.k_bias, nullptr, nullptr),
+                             call(L.v, E, KV, a.xn, E, a.v, KV, L.v_bias, nullptr, nullptr)};
+    if (launch_rmsnorm_rows(a.x, L.attn_norm, a.xn, E, T, eps) || gemv_batch3_launch(qkv))
       return -1;
     // model.c:1019-1090: QK-norm, RoPE, fp16 append and attention per token
     const int rc =

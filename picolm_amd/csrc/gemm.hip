@@ -1,0 +1,659 @@
+// gemm.hip -- the batched GEMV (matmul_batch, tensor.c:322-366) on the fp32
+// matrix cores, bit-identical to the single-vector kernel's exact order.
+//
+// The reference's dot products keep eight running sums per block (one per
+// AVX2 lane), each a chain of fused multiply-adds over the block's elements
+// 8s + j, and add the eight as hsum_avx2 does.  v_mfma_f32_16x16x4_f32 is
+// four such steps for 16 tokens x 16 rows at once: its K index is a chain of
+// correctly rounded fused multiply-adds in increasing k, subnormals kept
+// (checked on the device against fmaf on 0.5 M results per value range), so
+// with k = s one instruction per j forms a Q4_K sub-block's running sum j
+// from zero.  v_mfma_f32_16x16x1_4b_f32 (four independent 16 x 16 tiles, one
+// step each) forms four of a Q6_K group's running sums in two steps, or the
+// four rounded products of a Q8_0 block's lane.  A weight is then converted
+// to fp32 once per 16 or 32 tokens instead of once per token, and only the
+// adds between the running sums, the scales and the block chain stay on the
+// VALU.
+//
+// What bounds it: the fp32 MFMA and the VALU share one pipe (measured: a
+// 16x16x4 takes 32 cycles, and VALU instructions between them add their 4
+// cycles each), so a 16 x 16 tile of a 64-element Q4_K unit costs 16 x 32
+// MFMA cycles + ~150 x 4 VALU cycles (88 of them the exact order's own adds
+// and products).  TinyLlama's 128-token prompt, us a launch before (the VALU
+// kernel) and now: gate/up pair (5632 x 2048 Q4_K twice) 340 -> 96, down (2048 x
+// 5632 Q6_K) 287 -> 75, o 70 -> 25, q, k and v 102 in three launches -> 31 in
+// one; the whole prompt 18.1 -> 5.8 ms.  Set aside: x straight from the caches
+// instead of LDS (Q4_K 11264 x 2048, 128 tokens: 136 us against 96, Q6_K 387
+// against 130: the vector memory path handles the 16 tokens' lines one by
+// one); two token tiles a wave (88 against 94 us on that shape, slower below it).
+#include <algorithm>
+#include <type_traits>
+
+#include "gemv_formats.h"
+#include "plh_internal.h"
+
+using namespace plh;
+
+namespace {
+
+constexpr int kMT = 16;         // tokens and rows of one MFMA tile
+constexpr int kSubPitch = 36;   // staged floats per 32 elements of x (4 of padding)
+
+// x is staged in chunks: 256 elements, or 128 where the exchanged terms (KW 2)
+// would otherwise take the LDS of a second workgroup.  Staged floats per
+// token: a pitch of 4 mod 16 floats, so that 16 tokens' 16-byte reads hit
+// different banks.
+template <int KW>
+struct Chunk {
+  static constexpr int K = KW == 2 ? 128 : 256, U = K / 64;
+  static constexpr int kTokPitch = K / 32 * kSubPitch + 4;
+  static constexpr int kXs = kMT * kTokPitch;   // floats of a buffer
+  static constexpr int kSums = K / 32 * kMT;    // its sub-block sums [sub][token]
+};
+
+__device__ __forceinline__ float4_t mfma_f32_k4(float a, float b) {
+  const float4_t z = {0.f, 0.f, 0.f, 0.f};
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, z, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16_t mfma_f32_4b(float a, float b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+}
+
+// Byte b of a word as a float (plain C, so that the compiler sees every
+// operand the MFMAs read): v_cvt_f32_ubyte0..3.
+__device__ __forceinline__ float byte_f(uint32_t w, int b) {
+  return (float)((w >> (8 * b)) & 0xFFu);
+}
+
+// Keeps a masked word whole: without it the compiler extracts every nibble
+// with its own shift and mask instead of converting the word's bytes.
+__device__ __forceinline__ uint32_t whole(uint32_t w) {
+  asm("" : "+v"(w));
+  return w;
+}
+
+// 16 consecutive elements of x: one thread's share of a staged chunk, or a
+// lane's operand of one unit (64 elements) and token tile.
+struct XV {
+  float4_t f[4];
+};
+
+__device__ __forceinline__ float4_t ld4v(const float* p) { return *(const float4_t*)p; }
+
+// Makes the MFMAs that read x wait for v: without it the compiler starts
+// every tile of a chunk at once and runs out of registers.
+__device__ __forceinline__ void after(XV& x, float4_t& v) {
+  asm("" : "+v"(x.f[0]), "+v"(x.f[1]), "+v"(x.f[2]), "+v"(x.f[3]), "+v"(v));
+}
+
+// The formats.  Lane l = 16 s + c of a wave holds weight row c of the tile and
+// token c, the k = s (or tile s) operands; results are tokens 4 s .. 4 s + 3 of
+// row c.  Raw, load: the packed weights of one unit; W, weights: its fp32
+// operands and block scales; stage: 16 elements of x as the lanes read them;
+// load_x: a lane's operand, xt the staged unit of its token; terms: the unit's
+// kUnitTerms chained terms, sums the sub-block sums of x (kSums) at token 4 s
+// of the unit's first sub-block, sp floats per sub-block.
+struct Q4KM {
+  static constexpr int kUnitTerms = 1;
+  static constexpr bool kSums = true;
+  static constexpr bool kHalf = false;
+  struct Raw {
+    uint4 hdr;
+    uint2 q;  // bytes 8 s .. 8 s + 7 of the unit's 32
+  };
+  struct W {
+    float lo[8], hi[8];
+    float d1, m1, d2, m2;
+  };
+  static __device__ __forceinline__ void load(const GemvArgs& a, const uint8_t* w, int row, int s,
+                                              int unit, Raw& r) {
+    const uint32_t i = (uint32_t)row * a.nb * 4 + unit;
+    r.hdr = ld<uint4>(w, a.off0 + (i >> 2) * 16);
+    r.q = ld<uint2>(w, (s < 2 ? a.off1 : a.off2) + i * 16 + 8 * (s & 1));
+  }
+  static __device__ __forceinline__ void weights(const Raw& r, int u, int, W& w) {
+    const uint32_t q[2] = {r.q.x, r.q.y};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t lo = whole(q[h] & 0x0F0F0F0Fu), hi = whole((q[h] >> 4) & 0x0F0F0F0Fu);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) w.lo[4 * h + b] = byte_f(lo, b), w.hi[4 * h + b] = byte_f(hi, b);
+    }
+    // scales and mins of sub-blocks 2u, 2u + 1 (quant.c:82-91), u uniform
+    uint32_t sc, mn;
+    if (u < 2) {
+      sc = r.hdr.y & 0x3F3F3F3Fu;
+      mn = r.hdr.z & 0x3F3F3F3Fu;
+    } else {
+      sc = (r.hdr.w & 0x0F0F0F0Fu) | ((r.hdr.y >> 2) & 0x30303030u);
+      mn = ((r.hdr.w >> 4) & 0x0F0F0F0Fu) | ((r.hdr.z >> 2) & 0x30303030u);
+    }
+    sc >>= 16 * (u & 1);
+    mn >>= 16 * (u & 1);
+    const float dd = f16_bits_to_f32((uint16_t)(r.hdr.x & 0xFFFFu));
+    const float dmin = f16_bits_to_f32((uint16_t)(r.hdr.x >> 16));
+    w.d1 = dd * byte_f(sc, 0), w.m1 = dmin * byte_f(mn, 0);
+    w.d2 = dd * byte_f(sc, 1), w.m2 = dmin * byte_f(mn, 1);
+  }
+  static __device__ __forceinline__ void stage(const XV& x, float* dst) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(float4_t*)(dst + 4 * i) = x.f[i];
+  }
+  // x[8 s .. 8 s + 7] of both sub-blocks
+  static __device__ __forceinline__ void load_x(const float* xt, int s, XV& x) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x.f[i] = ld4v(xt + kSubPitch * (i >> 1) + 8 * s + 4 * (i & 1));
+  }
+  // the running sums of 32 elements, added as hsum_avx2 adds them
+  static __device__ __forceinline__ float4_t dot32(const float4_t& x0, const float4_t& x1,
+                                                   const float (&w)[8]) {
+    const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    float4_t v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = mfma_f32_k4(xv[j], w[j]);
+    return ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
+  }
+  static __device__ __forceinline__ void terms(const W& w, const XV& x, const float* sums, int sp,
+                                               float4_t* t) {
+    const float4_t x1 = *(const float4_t*)sums, x2 = *(const float4_t*)(sums + sp);
+    const float4_t q1 = dot32(x.f[0], x.f[1], w.lo);
+    const float4_t q2 = dot32(x.f[2], x.f[3], w.hi);
+    t[0] = ((w.d1 * q1 - w.m1 * x1) + w.d2 * q2) - w.m2 * x2;
+  }
+};
+
+struct Q6KM {
+  static constexpr int kUnitTerms = 4;
+  static constexpr bool kSums = false;
+  static constexpr bool kHalf = false;
+  struct Raw {
+    uint4 q[3];   // L0, L1, H words of the unit's four groups
+    uint32_t sc;  // their int8 scales
+    uint32_t d;
+  };
+  struct W {
+    float f[4][4];  // [group][element s + 4 e]
+    float ds[4];
+  };
+  static __device__ __forceinline__ void load(const GemvArgs& a, const uint8_t* w, int row, int,
+                                              int unit, Raw& r) {
+    const uint32_t i = (uint32_t)row * a.nb * 4 + unit;
+    const uint32_t offs[3] = {a.off0, a.off1, a.off2};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) r.q[p] = ld<uint4>(w, offs[p] + i * 16);
+    r.sc = ld<uint32_t>(w, a.scales_off + i * 4);
+    r.d = ld<uint16_t>(w, a.d_off + (i >> 2) * 2);
+  }
+  // byte s of the four groups' words, group g in byte g
+  static __device__ __forceinline__ uint32_t gather(const uint4& w, int s) {
+    const uint32_t sel = 0x0C0C0400u + 0x0101u * (uint32_t)s;
+    const uint32_t a = __builtin_amdgcn_perm(w.y, w.x, sel);
+    const uint32_t b = __builtin_amdgcn_perm(w.w, w.z, sel);
+    return a | (b << 16);
+  }
+  static __device__ __forceinline__ void weights(const Raw& r, int, int s, W& w) {
+    const uint32_t m4 = 0x0F0F0F0Fu, m30 = 0x30303030u;
+    const uint32_t L0 = gather(r.q[0], s), L1 = gather(r.q[1], s), H = gather(r.q[2], s);
+    const uint32_t v[4] = {(L0 & m4) | ((H << 4) & m30), ((L0 >> 4) & m4) | ((H << 2) & m30),
+                           (L1 & m4) | (H & m30), ((L1 >> 4) & m4) | ((H >> 2) & m30)};
+    const float dd = f16_bits_to_f32((uint16_t)(r.d & 0xFFFFu));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w.f[g][e] = byte_f(v[e], g) - 32.0f;
+      w.ds[g] = dd * sbyte(r.sc, g);
+    }
+  }
+  // elements e, 4 + e, 8 + e, 12 + e of the group side by side: lane s reads
+  // its four in one vector
+  static __device__ __forceinline__ void stage(const XV& x, float* dst) {
+    const float* e = (const float*)x.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *(float4*)(dst + 4 * i) = make_float4(e[i], e[4 + i], e[8 + i], e[12 + i]);
+  }
+  static __device__ __forceinline__ void load_x(const float* xt, int s, XV& x) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      x.f[g] = ld4v(xt + kSubPitch * (g >> 1) + 16 * (g & 1) + 4 * s);
+  }
+  static __device__ __forceinline__ void terms(const W& w, const XV& x, const float*, int,
+                                               float4_t* t) {
+    const f32x16_t z = {};
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      // running sum j: element j fused onto the product of element 8 + j
+      f32x16_t a = mfma_f32_4b(x.f[g].z, w.f[g][2], z), b = mfma_f32_4b(x.f[g].w, w.f[g][3], z);
+      a = mfma_f32_4b(x.f[g].x, w.f[g][0], a);
+      b = mfma_f32_4b(x.f[g].y, w.f[g][1], b);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float h = ((a[v] + b[v]) + (a[8 + v] + b[8 + v])) +
+                        ((a[4 + v] + b[4 + v]) + (a[12 + v] + b[12 + v]));
+        t[g][v] = w.ds[g] * h;
+      }
+    }
+  }
+};
+
+struct Q80M {
+  static constexpr int kUnitTerms = 2;
+  static constexpr bool kSums = false;
+  static constexpr bool kHalf = true;  // a row's last unit may be one block
+  struct Raw {
+    uint2 q[2];  // bytes 8 s .. 8 s + 7 of the unit's two blocks
+    uint32_t d[2];
+  };
+  struct W {
+    float f[2][8];
+    float d[2];
+  };
+  static __device__ __forceinline__ void load(const GemvArgs& a, const uint8_t* w, int row, int s,
+                                              int unit, Raw& r) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // blocks past the row's end re-read its last one (their terms are not used)
+      const uint32_t blk = (uint32_t)row * a.nb + min(2 * unit + h, a.nb - 1);
+      r.q[h] = ld<uint2>(w, (s < 2 ? a.off0 : a.off1) + blk * 16 + 8 * (s & 1));
+      r.d[h] = ld<uint16_t>(w, a.d_off + blk * 2);
+    }
+  }
+  static __device__ __forceinline__ void weights(const Raw& r, int, int, W& w) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        w.f[h][b] = sbyte(r.q[h].x, b), w.f[h][4 + b] = sbyte(r.q[h].y, b);
+      w.d[h] = f16_bits_to_f32((uint16_t)(r.d[h] & 0xFFFFu));
+    }
+  }
+  static __device__ __forceinline__ void stage(const XV& x, float* dst) { Q4KM::stage(x, dst); }
+  static __device__ __forceinline__ void load_x(const float* xt, int s, XV& x) {
+    Q4KM::load_x(xt, s, x);
+  }
+  static __device__ __forceinline__ void terms(const W& w, const XV& x, const float*, int,
+                                               float4_t* t) {
+    const f32x16_t z = {};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float4_t x0 = x.f[2 * h], x1 = x.f[2 * h + 1];
+      if (h) asm("" : "+v"(x0), "+v"(x1), "+v"(t[0]));  // as after()
+      const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      float4_t acc[8];
+      f32x16_t p = mfma_f32_4b(xv[0], w.f[h][0], z);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        // p: the rounded products of elements k, 8 + k, 16 + k, 24 + k; the
+        // next four are multiplied while these are added
+        f32x16_t n = p;
+        if (k < 7) {
+          n = mfma_f32_4b(xv[k + 1], w.f[h][k + 1], z);
+          asm("" : "+v"(p), "+v"(n));
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[k][v] = (p[v] + p[4 + v]) + (p[8 + v] + p[12 + v]);
+        p = n;
+      }
+      t[h] = w.d[h] *
+             (((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7])));
+    }
+  }
+};
+
+// sum_x of a 32-element sub-block (quant.c:433, as Q4K::load_x): running sum k
+// is (x[k] + x[8+k]) + (x[16+k] + x[24+k]), the pairs in this lane (the even
+// lane of a pair holds elements 0-15, the odd one 16-31).
+__device__ __forceinline__ float sub_sum(const XV& x) {
+  const float* e = (const float*)x.f;
+  float t[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float p = 0.0f + (e[k] + e[8 + k]);
+    const int q = __builtin_amdgcn_mov_dpp(__float_as_int(p), 0xB1, 0xF, 0xF, true);  // lane ^ 1
+    t[k] = p + __int_as_float(q);
+  }
+  return hsum8(t);
+}
+
+// LDS floats of a workgroup: two buffers of staged x and its sums, two of the
+// terms that waves of one row tile exchange (KW > 1).
+template <class F, int KW>
+constexpr int x_floats() {
+  return Chunk<KW>::kXs + (F::kSums ? Chunk<KW>::kSums : 0);
+}
+template <class F, int KW, int M>
+constexpr int term_floats() {
+  return KW == 1 ? 0 : 4 / KW * Chunk<KW>::U * F::kUnitTerms * M * 4 * 64;
+}
+template <class F, int KW, bool PAIR>
+constexpr size_t lds_bytes() {
+  return sizeof(float) * 2 * (size_t)(x_floats<F, KW>() + term_floats<F, KW, PAIR ? 2 : 1>());
+}
+
+// One workgroup: 16 tokens x (4 / KW) * 16 rows (of two matrices for a gate/up
+// pair).  The four waves take row tiles of their own (KW 1), or KW waves share
+// a row tile: each forms the terms of a KW-th of a chunk's units into LDS,
+// then chains a KW-th of the tile's sums over the chunk's terms, in block
+// order.  One barrier per chunk; the next chunk's x, the next unit's operand
+// and the weights of the next two units are in flight meanwhile.
+template <class F, int KW, bool PAIR>
+__device__ __forceinline__ void gemm_body(const GemvArgs& a, const BatchShape& b, int r_tile,
+                                          int t_tile, float* lds) {
+  using C = Chunk<KW>;
+  constexpr int RW = 4 / KW, M = PAIR ? 2 : 1;
+  constexpr int S = 4 / KW;  // sums per lane and matrix
+  constexpr int TU = F::kUnitTerms, UW = C::U / KW;  // a wave's units of a chunk
+  constexpr int XF = x_floats<F, KW>(), TF = term_floats<F, KW, M>();
+  static_assert(UW * KW == C::U, "a chunk's units divide among the waves");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, s = lane >> 4;
+  const int kw = wave % KW, rw = wave / KW;
+  const int r = (r_tile * RW + rw) * kMT + c;
+  const int row = min(r, a.d - 1);
+  const int tk0 = t_tile * kMT;
+  const int units = (a.n + 63) / 64;  // the last may be half (Q8_0)
+  const int chunks = (a.n + C::K - 1) / C::K;
+  // staging: thread p takes 16-element piece p % PP of token p / PP; pieces
+  // past the row's end re-read its last one, tokens past the prompt's its last
+  // (not used)
+  constexpr int PP = C::K / 16;
+  const int stok = tid / PP, piece = tid % PP;
+  const bool stager = tid < PP * kMT;
+  const float* xsrc = a.x + (size_t)min(tk0 + stok, b.n_tok - 1) * b.x_stride;
+  const int xdst = stok * C::kTokPitch + (piece >> 1) * kSubPitch + 16 * (piece & 1);
+  XV xg;
+  auto fetch_x = [&](int chunk) {
+    if (!stager) return;
+    const float* p = xsrc + min(chunk * C::K + 16 * piece, a.n - 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xg.f[i] = ld4v(p + 4 * i);
+  };
+  auto stage_x = [&](float* buf) {
+    if (!stager) return;
+    F::stage(xg, buf + xdst);
+    if constexpr (F::kSums) {
+      const float v = sub_sum(xg);
+      if ((piece & 1) == 0) buf[C::kXs + (piece >> 1) * kMT + stok] = v;
+    }
+  };
+  // KW 1: tokens 4 s .. 4 s + 3 of row c; else this wave's S of them
+  float4_t sum[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) sum[m] = float4_t{0.f, 0.f, 0.f, 0.f};
+  // unit k (0 .. 2 UW - 1) of this wave, counted from chunk on
+  auto unit_at = [&](int chunk, int k) { return (chunk + k / UW) * C::U + kw * UW + k % UW; };
+  typename F::Raw raw[2][M];
+  auto load_w = [&](int unit, typename F::Raw(&w)[M]) {
+    F::load(a, a.w, row, s, min(unit, units - 1), w[0]);
+    if constexpr (PAIR) F::load(a, a.w2, row, s, min(unit, units - 1), w[1]);
+  };
+  // One chunk; with one unit a chunk its weights are in raw[P], else a wave's
+  // even units' are in raw[0] and its odd ones' in raw[1].
+  auto body = [&](int chunk, auto par) {
+    constexpr int P = decltype(par)::value;
+    float* xs = lds + (chunk & 1) * XF;
+    float* xch = lds + 2 * XF + (chunk & 1) * TF;
+    const bool more = chunk + 1 < chunks;
+    if (more) fetch_x(chunk + 1);
+    const float* xt = xs + c * C::kTokPitch + kw * UW * 2 * kSubPitch;
+    XV xn;
+    F::load_x(xt, s, xn);
+    // unit k of the wave's UW, its weights in rk
+    auto step = [&](int k, typename F::Raw(&rk)[M]) {
+      const int ku = kw * UW + k, unit = chunk * C::U + ku;
+      typename F::W w[M];
+#pragma unroll
+      for (int m = 0; m < M; ++m) F::weights(rk[m], unit & 3, s, w[m]);
+      load_w(unit_at(chunk, k + 2), rk);
+      XV x = xn;
+      // after the chunk's last unit: read again, not used
+      F::load_x(xt + min(k + 1, UW - 1) * 2 * kSubPitch, s, xn);
+      const float* st = xs + C::kXs + 2 * ku * kMT + 4 * s;
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        float4_t t[TU];
+        F::terms(w[m], x, st, kMT, t);
+        if constexpr (KW == 1) {
+#pragma unroll
+          for (int g = 0; g < TU; ++g)
+            if (!F::kHalf || unit * TU + g < a.terms) sum[m] = sum[m] + t[g];
+          if constexpr (M > 1) after(m + 1 < M ? x : xn, sum[m]);
+        } else {
+          float* o = xch + ((rw * C::U + ku) * TU * M + m) * 256 + 4 * lane;
+#pragma unroll
+          for (int g = 0; g < TU; ++g) *(float4_t*)(o + g * M * 256) = t[g];
+          if constexpr (M > 1) after(m + 1 < M ? x : xn, t[TU - 1]);
+        }
+      }
+    };
+    if constexpr (UW == 1) {
+      step(0, raw[P]);
+    } else {
+#pragma unroll 1
+      for (int k = 0; k < UW; k += 2) {
+        step(k, raw[0]);
+        step(k + 1, raw[1]);
+      }
+    }
+    if (more) stage_x(lds + ((chunk + 1) & 1) * XF);
+    __syncthreads();
+    if constexpr (KW > 1) {
+      const int left = a.terms - chunk * C::U * TU;
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const float* o = xch + (rw * C::U * TU * M + m) * 256 + 4 * lane + kw * S;
+#pragma unroll
+        for (int g = 0; g < C::U * TU; ++g) {
+          if (F::kHalf && g >= left) break;
+          if constexpr (S == 1) {
+            sum[m][0] = sum[m][0] + o[g * M * 256];
+          } else {
+            const float2 v = *(const float2*)(o + g * M * 256);
+            sum[m][0] = sum[m][0] + v.x;
+            sum[m][1] = sum[m][1] + v.y;
+          }
+        }
+      }
+    }
+  };
+  fetch_x(0);
+  load_w(unit_at(0, 0), raw[0]);
+  load_w(unit_at(0, 1), raw[1]);
+  stage_x(lds);
+  __syncthreads();
+  if constexpr (UW == 1) {
+#pragma unroll 1
+    for (int chunk = 0; chunk < chunks; chunk += 2) {
+      body(chunk, std::integral_constant<int, 0>{});
+      if (chunk + 1 < chunks) body(chunk + 1, std::integral_constant<int, 1>{});
+    }
+  } else {
+#pragma unroll 1
+    for (int chunk = 0; chunk < chunks; ++chunk) body(chunk, std::integral_constant<int, 0>{});
+  }
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    const int tok = tk0 + 4 * s + kw * S + i;
+    if (r >= a.d || tok >= b.n_tok) continue;
+    const size_t o = (size_t)tok * b.out_stride + r;
+    float v = sum[0][i];
+    if constexpr (PAIR) {
+      a.out[o] = silu(v) * sum[M - 1][i];
+    } else {
+      if (a.bias_mode == 1) v = v + a.bias[r];
+      if (a.bias_mode == 2) v = v + 0.0f;
+      if (a.gate) v = silu(a.gate[o]) * v;
+      if (a.resid) v = a.resid[o] + v;
+      a.out[o] = v;
+    }
+  }
+}
+
+// Workgroup id -> row tile and token tile: the token tiles of a row tile share
+// an XCD (ids congruent mod 8) and its L2, so its weights come from HBM about
+// once.  False past the last row tile.
+__device__ __forceinline__ bool tile_of(int row_tiles, int tok_tiles, int& r_tile, int& t_tile) {
+  const int kb = blockIdx.x >> 3;
+  r_tile = (kb / tok_tiles) * 8 + (blockIdx.x & 7);
+  t_tile = kb % tok_tiles;
+  return r_tile < row_tiles;
+}
+
+template <class F, int KW, bool PAIR>
+__global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemvArgs a, BatchShape b) {
+  extern __shared__ __align__(16) float lds[];
+  int r_tile, t_tile;
+  if (tile_of(b.row_tiles, b.tok_tiles, r_tile, t_tile))
+    gemm_body<F, KW, PAIR>(a, b, r_tile, t_tile, lds);
+}
+
+// Up to three matrices over the same x in one launch (q, k and v), the row
+// tiles of each a range of the grid's: a small matrix alone leaves most CUs
+// idle.
+struct MultiBatch {
+  GemvArgs seg[3];
+  BatchShape shape[3];  // row_tiles: of the segment
+  int qtype[3];
+  int tile1, tile2, row_tiles;  // first tiles of segments 1 and 2, all tiles
+};
+
+template <int KW>
+__global__ __launch_bounds__(kThreads) void gemm_mfma_multi_kernel(MultiBatch m) {
+  extern __shared__ __align__(16) float lds[];
+  int r_tile, t_tile;
+  if (!tile_of(m.row_tiles, m.shape[0].tok_tiles, r_tile, t_tile)) return;
+  const int i = (r_tile >= m.tile1) + (r_tile >= m.tile2);
+  r_tile -= i == 2 ? m.tile2 : i == 1 ? m.tile1 : 0;
+  switch (m.qtype[i]) {
+    case kTypeQ4K: gemm_body<Q4KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds); break;
+    case kTypeQ8_0:  // never with KW 1 (waves_per_tile)
+      if constexpr (KW > 1)
+        gemm_body<Q80M, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
+      break;
+    default: gemm_body<Q6KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds); break;
+  }
+}
+
+int cu_count() { return ctx().num_cus > 0 ? ctx().num_cus : 256; }
+
+// Waves per row tile, from the launch's 16 x 16 tiles (a pair's count once):
+// the most that still adds waves to idle SIMDs.  Measured, us at n = 2048,
+// KW 4 / 2 / 1: Q4_K 256 tiles 11.2 / 18.6 / 23.9, 1024 26.8 / 25.7 / 25.4,
+// 1408 35 / 32 / 37, 5632 114 / 95 / 94; Q6_K 256 13.6 / 21 / 28, 1024 36 /
+// 32 / 30, 5632 179 / 142 / 137.  Q8_0's products keep four tiles of
+// registers each and spill the unsplit form: 5632 tiles 179 / 156 / 213.
+int waves_per_tile(long tiles, bool q8) {
+  const int cus = cu_count();
+  if (tiles < 4L * cus) return 4;
+  return tiles < 8L * cus || q8 ? 2 : 1;
+}
+
+BatchShape shape_of(const GemvArgs& a, int n_tok, int x_stride, int out_stride, int kw) {
+  BatchShape b{};
+  b.n_tok = n_tok;
+  b.x_stride = x_stride;
+  b.out_stride = out_stride;
+  b.row_tiles = (a.d + kMT * (4 / kw) - 1) / (kMT * (4 / kw));
+  b.tok_tiles = (n_tok + kMT - 1) / kMT;
+  return b;
+}
+
+unsigned grid_of(int row_tiles, int tok_tiles) {
+  return 8u * (unsigned)((row_tiles + 7) / 8) * (unsigned)tok_tiles;
+}
+
+long tiles_of(const GemvArgs& a, int n_tok) {
+  return (long)((a.d + kMT - 1) / kMT) * ((n_tok + kMT - 1) / kMT);
+}
+
+template <class F, int KW>
+void launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
+  const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(kThreads);
+  if (pair)
+    hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, true>), grid, block, (lds_bytes<F, KW, true>()),
+                       st, a, b);
+  else
+    hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, false>), grid, block, (lds_bytes<F, KW, false>()),
+                       st, a, b);
+}
+template <class F>
+void launch_f(int kw, bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
+  if (kw == 4) {
+    launch_k<F, 4>(pair, a, b, st);
+  } else if (F::kHalf || kw == 2) {  // Q8_0: waves_per_tile has no 1
+    launch_k<F, 2>(pair, a, b, st);
+  } else {
+    if constexpr (!F::kHalf) launch_k<F, 1>(pair, a, b, st);
+  }
+}
+
+template <int KW>
+void launch_multi(const MultiBatch& m, hipStream_t st) {
+  size_t lds = std::max(lds_bytes<Q4KM, KW, false>(), lds_bytes<Q6KM, KW, false>());
+  if constexpr (KW > 1) lds = std::max(lds, lds_bytes<Q80M, KW, false>());
+  hipLaunchKernelGGL((gemm_mfma_multi_kernel<KW>), dim3(grid_of(m.row_tiles, m.shape[0].tok_tiles)),
+                     dim3(kThreads), lds, st, m);
+}
+
+}  // namespace
+
+namespace plh {
+
+// The estimates, in us, are fits to measured times of both kernels (n 256 to
+// 11008, d 65 to 11264, 2 to 128 tokens, warm): the VALU kernel's 6 to 8 plus
+// its work per weight and token; here a wave's chain of units (0.26 a unit
+// with four waves on a row, whatever the number of rows) or, with the chip
+// full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and 2 / 4 / 17
+// / 128 tokens the two take 8.7 / 12.2 / 20 / 70 and 10.9 / 10.9 / 11.2 / 25 us,
+// at n = 11008, d = 129 and 40 tokens 18.4 and 48.6.
+bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
+  const double w = 1e-6 * a.n * (double)a.d * (pair ? 2 : 1);
+  const bool q4 = qtype == kTypeQ4K, q8 = qtype == kTypeQ8_0;
+  const double valu = (q8 ? 6.0 : 8.0) + w * n_tok * (q4 ? 0.12 : q8 ? 0.125 : 0.22);
+  const double work = w * ((n_tok + kMT - 1) / kMT * kMT) * (q4 ? 0.032 : q8 ? 0.053 : 0.046);
+  const double chain = 0.26 * ((a.n + 63) / 64) * (pair ? 2 : 1);
+  return 2.5 + std::max(chain, work) < valu;
+}
+
+int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride) {
+  const int kw = waves_per_tile(tiles_of(a, n_tok), qtype == kTypeQ8_0);
+  const BatchShape b = shape_of(a, n_tok, x_stride, out_stride, kw);
+  hipStream_t st = ctx().stream;
+  if (qtype == kTypeQ4K)
+    launch_f<Q4KM>(kw, pair, a, b, st);
+  else if (qtype == kTypeQ8_0)
+    launch_f<Q80M>(kw, pair, a, b, st);
+  else
+    launch_f<Q6KM>(kw, pair, a, b, st);
+  return check_hip(hipGetLastError(), "gemm_mfma_kernel launch");
+}
+
+int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride,
+                    const int* out_stride) {
+  MultiBatch m{};
+  long tiles = 0;
+  bool q8 = false;
+  for (int i = 0; i < 3; ++i) {
+    tiles += tiles_of(a[i], n_tok);
+    q8 = q8 || qtype[i] == kTypeQ8_0;
+  }
+  const int kw = waves_per_tile(tiles, q8);
+  for (int i = 0; i < 3; ++i) {
+    m.seg[i] = a[i];
+    m.qtype[i] = qtype[i];
+    m.shape[i] = shape_of(a[i], n_tok, x_stride, out_stride[i], kw);
+  }
+  m.tile1 = m.shape[0].row_tiles;
+  m.tile2 = m.tile1 + m.shape[1].row_tiles;
+  m.row_tiles = m.tile2 + m.shape[2].row_tiles;
+  if (kw == 1)
+    launch_multi<1>(m, ctx().stream);
+  else if (kw == 2)
+    launch_multi<2>(m, ctx().stream);
+  else
+    launch_multi<4>(m, ctx().stream);
+  return check_hip(hipGetLastError(), "gemm_mfma_multi_kernel launch");
+}
+
+}  // namespace plh

@@ -24,6 +24,7 @@
 
 #include "attn_common.h"
 #include "attn_decode_dev.h"
+#include "gemv_formats.h"
 #include "picolm_hip.h"
 #include "plh_internal.h"
 
@@ -36,10 +37,6 @@ int g_gemv_exact = 0;
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kTypeQ8_0 = 8, kTypeQ4K = 12, kTypeQ6K = 14;
-constexpr size_t kPlaneAlign = 256;
-constexpr size_t kMaxPacked = (size_t)1 << 31;  // 32-bit plane offsets
 constexpr int kMaxNormN = kGemvNormMax;          // squares + staged x within 64 KiB of LDS
 constexpr int kNormPrefetch = 16;                // x elements per thread loaded up front
 
@@ -148,51 +145,6 @@ void pack_rows(int qtype, const Layout& L, int d, const uint8_t* src, uint8_t* d
   }
 }
 
-struct GemvArgs {
-  const uint8_t* w;     // packed matrix
-  const float* x;       // [n]
-  float* out;           // [d]
-  int d;
-  int nb;               // blocks per row
-  int units;            // lane units per row
-  int uspan;            // units covered by one pass of the threads (<= 256)
-  int row_par;          // rows worked side by side (kThreads / uspan)
-  int unit_iters;       // passes over the units
-  int rows_per_wg;      // rows of one workgroup (row_par * rows per thread)
-  int terms;            // chained terms per row
-  int tpitch;           // LDS pitch of a row's terms
-  uint32_t off0, off1, off2, scales_off, d_off;  // plane offsets (bytes)
-  // Epilogue, in the reference's order (tensor.c:256-264, 605-657):
-  // v = dot; v = v + bias[i] (bias_mode 1) or v + 0.0f (bias_mode 2, a
-  // zero-filled bias); v = silu(gate[i]) * v; v = resid[i] + v.
-  const float* bias;
-  const float* gate;
-  const float* resid;
-  int bias_mode;
-  // Prologue (gemv_kernel<..., true>): x is rmsnorm(x, norm_w) of length n
-  // (tensor.c:425-492), formed by every workgroup itself.
-  const float* norm_w;
-  float norm_eps;
-  int n;
-  int xs_off;  // floats from the LDS base to the staged rmsnorm(x)
-  float* xn_out;  // workgroup 0 also stores rmsnorm(x) here (or null)
-  // Gate/up pair (gemv_body<..., true>): virtual row 2r is row r of w (gate),
-  // 2r + 1 row r of w2 (up, same type and shape); out[r] = silu(gate) * up.
-  const uint8_t* w2;
-};
-
-// tensor.c:605-609: x / (1 + expf(-x)).  expf is the device library's, not
-// glibc's (which is not correctly rounded), so results can differ from the
-// host's in the last place.
-__device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
-
-__device__ __forceinline__ float hsum8(const float (&v)[8]) {
-  const float a0 = v[0] + v[4], a1 = v[1] + v[5], a2 = v[2] + v[6], a3 = v[3] + v[7];
-  return (a0 + a2) + (a1 + a3);
-}
-
-__device__ __forceinline__ float4 ld4(const float* p) { return *(const float4*)p; }
-
 // The x operand as the formats read it, four elements at a time: the vector
 // itself, or its rmsnorm (x * scale) * w formed on the fly, rounded as the
 // reference's rmsnorm rounds it.
@@ -211,33 +163,6 @@ struct LdsX {
     return *(const float4*)(xs + xs_index(i));
   }
 };
-
-template <class T>
-__device__ __forceinline__ T ld(const uint8_t* w, uint32_t off) {
-  return *(const T*)(w + off);
-}
-
-// byte B of a word as a float, exact (v_cvt_f32_ubyteB: one instruction)
-template <int B>
-__device__ __forceinline__ float ubyte(uint32_t w) {
-  float r;
-  if constexpr (B == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(r) : "v"(w));
-  if constexpr (B == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(r) : "v"(w));
-  if constexpr (B == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(w));
-  if constexpr (B == 3) asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(w));
-  return r;
-}
-__device__ __forceinline__ float ubyte(uint32_t w, int b) {
-  switch (b) {
-    case 0: return ubyte<0>(w);
-    case 1: return ubyte<1>(w);
-    case 2: return ubyte<2>(w);
-    default: return ubyte<3>(w);
-  }
-}
-__device__ __forceinline__ float sbyte(uint32_t w, int b) {
-  return (float)(int)(int8_t)((w >> (8 * b)) & 0xFFu);
-}
 
 // ---- Q4_K: a unit is 64-element sub-block s = 4 * block + j ---------------
 struct Q4K {
@@ -624,21 +549,13 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, int wg, float* term
 // workgroup holds its rows' weights in registers and runs up to kTokTile
 // tokens over them; the token tiles of one row tile share an XCD (and its
 // L2), so the weights come from HBM about once per chunk.
-// Four tokens per workgroup measured fastest for a 128-token TinyLlama
-// prompt (1, 2, 3, 5, 6, 8 tokens: 28.6, 21.5, 20.4, 19.2, 22.2, 20.1 ms
-// against 18.3; 16 leave no room for the term buffer).
+// Used for few tokens and for few long rows (gemm_mfma_pays); the rest runs on
+// the matrix cores (gemm.hip).
 constexpr int kTokTile = 4;
 
-struct BatchArgs {
-  GemvArgs a;
-  int n_tok, x_stride, out_stride;  // tokens, floats between x rows / out rows
-  int row_tiles, tok_tiles;
-};
-
 template <class F, int RB, bool PAIR>
-__global__ __launch_bounds__(kThreads) void gemm_kernel(BatchArgs b) {
+__global__ __launch_bounds__(kThreads) void gemm_kernel(GemvArgs a, BatchShape b) {
   extern __shared__ __align__(16) float terms[];  // [row][token][tpitch]
-  const GemvArgs& a = b.a;
   const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
   const int r_tile = (k / b.tok_tiles) * 8 + xcd;
   const int t_tile = k % b.tok_tiles;
@@ -1503,57 +1420,69 @@ int launch_single(int qtype, bool pair, const GemvArgs& a0, int rows) {
 }
 
 template <class F, bool PAIR>
-void launch_batch(int rb, int grid, size_t lds, hipStream_t st, const BatchArgs& b) {
+void launch_batch(int rb, int grid, size_t lds, hipStream_t st, const GemvArgs& a,
+                  const BatchShape& b) {
   switch (rb) {
     case 1:
-      hipLaunchKernelGGL((gemm_kernel<F, 1, PAIR>), dim3(grid), dim3(kThreads), lds, st, b);
+      hipLaunchKernelGGL((gemm_kernel<F, 1, PAIR>), dim3(grid), dim3(kThreads), lds, st, a, b);
       break;
     case 2:
-      hipLaunchKernelGGL((gemm_kernel<F, 2, PAIR>), dim3(grid), dim3(kThreads), lds, st, b);
+      hipLaunchKernelGGL((gemm_kernel<F, 2, PAIR>), dim3(grid), dim3(kThreads), lds, st, a, b);
       break;
     default:
-      hipLaunchKernelGGL((gemm_kernel<F, 4, PAIR>), dim3(grid), dim3(kThreads), lds, st, b);
+      hipLaunchKernelGGL((gemm_kernel<F, 4, PAIR>), dim3(grid), dim3(kThreads), lds, st, a, b);
       break;
   }
 }
 
+// Rows per thread of the VALU kernel: the most (4, 2, 1) whose term buffer for
+// kTokTile tokens fits 64 KiB of LDS; 0 where none does (error set: such rows
+// are refused whichever kernel would run).
+int batch_rb(const GemvArgs& a, bool pair) {
+  if (a.norm_w) {
+    set_error("batched GEMV: no rmsnorm prologue (normalise the rows first)");
+    return 0;
+  }
+  int rb = 4;
+  while (rb > 1 && (size_t)a.row_par * rb * kTokTile * a.tpitch * sizeof(float) > 64 * 1024)
+    rb /= 2;
+  if (pair && (a.row_par * rb) % 2) rb *= 2;
+  if ((size_t)a.row_par * rb * kTokTile * a.tpitch * sizeof(float) > 64 * 1024) {
+    set_error("batched GEMV: row of %d weights too long for the term buffer", a.n);
+    return 0;
+  }
+  return rb;
+}
+
 // Batched launch over n_tok tokens (x rows x_stride apart, out rows
 // out_stride apart; gate and resid indexed like out).  No rmsnorm prologue.
+// The matrix cores (gemm.hip) except for few tokens or few long rows.
 int launch_batched(int qtype, bool pair, const GemvArgs& a0, int rows, int n_tok, int x_stride,
                    int out_stride) {
-  if (a0.norm_w) {
-    set_error("batched GEMV: no rmsnorm prologue (normalise the rows first)");
-    return -1;
-  }
-  BatchArgs b{};
-  b.a = a0;
-  // rows per thread: the most (4, 2, 1) whose term buffer for kTokTile tokens
-  // fits 64 KiB of LDS
-  int rb = 4;
-  while (rb > 1 &&
-         (size_t)b.a.row_par * rb * kTokTile * b.a.tpitch * sizeof(float) > 64 * 1024)
-    rb /= 2;
-  if (pair && (b.a.row_par * rb) % 2) rb *= 2;
-  const size_t lds = (size_t)b.a.row_par * rb * kTokTile * b.a.tpitch * sizeof(float);
-  if (lds > 64 * 1024) {
-    set_error("batched GEMV: row of %d weights too long for the term buffer", b.a.n);
-    return -1;
-  }
-  b.a.rows_per_wg = b.a.row_par * rb;
+  const int rb = batch_rb(a0, pair);
+  if (!rb) return -1;
+  if (gemm_mfma_pays(qtype, a0, n_tok, pair))
+    return gemm_mfma(qtype, pair, a0, n_tok, x_stride, out_stride);
+  GemvArgs a = a0;
+  a.rows_per_wg = a.row_par * rb;
+  const size_t lds = (size_t)a.rows_per_wg * kTokTile * a.tpitch * sizeof(float);
+  BatchShape b{};
   b.n_tok = n_tok;
   b.x_stride = x_stride;
   b.out_stride = out_stride;
-  b.row_tiles = (rows + b.a.rows_per_wg - 1) / b.a.rows_per_wg;
+  b.row_tiles = (rows + a.rows_per_wg - 1) / a.rows_per_wg;
   b.tok_tiles = (n_tok + kTokTile - 1) / kTokTile;
   const int grid = 8 * ((b.row_tiles + 7) / 8) * b.tok_tiles;
   hipStream_t st = ctx().stream;
   if (qtype == kTypeQ4K)
-    pair ? launch_batch<Q4K, true>(rb, grid, lds, st, b) : launch_batch<Q4K, false>(rb, grid, lds, st, b);
+    pair ? launch_batch<Q4K, true>(rb, grid, lds, st, a, b)
+         : launch_batch<Q4K, false>(rb, grid, lds, st, a, b);
   else if (qtype == kTypeQ8_0)
-    pair ? launch_batch<Q80, true>(rb, grid, lds, st, b) : launch_batch<Q80, false>(rb, grid, lds, st, b);
+    pair ? launch_batch<Q80, true>(rb, grid, lds, st, a, b)
+         : launch_batch<Q80, false>(rb, grid, lds, st, a, b);
   else
-    pair ? launch_batch<Q6K<4>, true>(rb, grid, lds, st, b)
-         : launch_batch<Q6K<4>, false>(rb, grid, lds, st, b);
+    pair ? launch_batch<Q6K<4>, true>(rb, grid, lds, st, a, b)
+         : launch_batch<Q6K<4>, false>(rb, grid, lds, st, a, b);
   return check_hip(hipGetLastError(), "gemm_kernel launch");
 }
 
@@ -1700,6 +1629,35 @@ int gemv_multi_launch(const GemvCall* g, int n) {
   else
     launch_multi<false>(rb, m.wg0[n], lds, ctx().stream, m);
   return check_hip(hipGetLastError(), "gemv_multi_kernel launch");
+}
+
+int gemv_batch3_launch(const GemvCall* g) {
+  if (!ctx().stream) {
+    set_error("plh_gemv: plh_init has not been called");
+    return -1;
+  }
+  GemvArgs a[3];
+  int qtype[3], out_stride[3];
+  bool together = true;
+  for (int s = 0; s < 3; ++s) {
+    if (g[s].x != g[0].x || g[s].n != g[0].n || g[s].n_tok != g[0].n_tok ||
+        g[s].x_stride != g[0].x_stride) {
+      set_error("gemv_batch3_launch: segments must share x");
+      return -1;
+    }
+    if (prepare(g[s], a[s])) return -1;
+    qtype[s] = g[s].qtype;
+    out_stride[s] = g[s].out_stride;
+    together = together && g[s].n_tok > 1;
+    if (g[s].n_tok > 1 && !batch_rb(a[s], false)) return -1;
+  }
+  // one launch where the matrix cores would run the largest of the three
+  if (!together || !gemm_mfma_pays(qtype[0], a[0], g[0].n_tok, false)) {
+    for (int s = 0; s < 3; ++s)
+      if (gemv_launch(g[s])) return -1;
+    return 0;
+  }
+  return gemm_mfma_multi(qtype, a, g[0].n_tok, g[0].x_stride, out_stride);
 }
 
 int qkv_attention_launch(const GemvCall* g, const DecodeArgs& d, int head_dim, unsigned* ctr,

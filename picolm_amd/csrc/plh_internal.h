@@ -103,6 +103,9 @@ int gemv_launch(const GemvCall& g);
 // Up to three GEMVs over the same x (and the same rmsnorm prologue, if any)
 // in one launch: the q, k and v projections.
 int gemv_multi_launch(const GemvCall* g, int n);
+// Three batched GEMVs (n_tok > 1) over the same x: one launch where the matrix
+// cores run them, else one each.
+int gemv_batch3_launch(const GemvCall* g);
 // hb = silu(gate(x)) * up(x) in one launch (model.c:906-916), gate and up of
 // the same type and shape and the same rmsnorm prologue (or none); out =
 // up.out.

@@ -1,0 +1,85 @@
+"""The batched GEMV (plh_matmul_batch) on the matrix cores, bit for bit against
+the oracle's vec_dot per (row, token): every waves-per-row-tile form (chosen by
+the number of 16 x 16 tiles: below 1024 four waves, below 2048 two, else one),
+rows and tokens that leave partial tiles, rows of one unit, of one chunk, of an
+odd number of blocks (Q8_0's half unit), and the shapes that stay on the VALU
+kernel.  Subnormal and huge activations, and infinities and NaNs that must stay
+in their token."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from picolm_amd import gemv as G
+from picolm_amd import synth as S
+
+pytestmark = pytest.mark.gpu
+
+Q4, Q6, Q8 = G.TYPE_Q4_K, G.TYPE_Q6_K, G.TYPE_Q8_0
+
+
+def batch(P, W, X):
+    dx, out = P.DeviceBuffer.from_numpy(X), P.DeviceBuffer(4 * X.shape[0] * W.d)
+    P.check(P.lib.plh_matmul_batch(W.qtype, W.n, W.d, C.c_void_p(W.ptr), C.c_void_p(dx.ptr),
+                                   X.shape[0], C.c_void_p(out.ptr)), "plh_matmul_batch")
+    got = out.download(np.float32, (X.shape[0], W.d))
+    dx.free()
+    out.free()
+    return got
+
+
+def assert_bits(got, want, what):
+    bad = np.flatnonzero(got.view(np.uint32) != want.view(np.uint32))
+    # a NaN's payload is not part of the contract
+    bad = bad[~(np.isnan(got.ravel()[bad]) & np.isnan(want.ravel()[bad]))]
+    assert bad.size == 0, (what, bad[:8], got.ravel()[bad[:4]], want.ravel()[bad[:4]])
+
+
+@pytest.mark.parametrize("qtype,n,d,tokens", [
+    (Q4, 256, 1, 16), (Q4, 256, 77, 33), (Q4, 512, 16, 15), (Q4, 768, 65, 17), (Q4, 2048, 200, 5),
+    (Q6, 256, 3, 19), (Q6, 512, 33, 16), (Q6, 1280, 130, 31), (Q6, 2048, 64, 6),
+    (Q8, 32, 5, 20), (Q8, 64, 16, 16), (Q8, 96, 100, 37), (Q8, 288, 17, 18), (Q8, 1056, 64, 33),
+    (Q4, 256, 8200, 32), (Q6, 256, 8200, 32), (Q8, 160, 8200, 32),     # two waves a tile
+    (Q4, 512, 16400, 31), (Q6, 256, 16400, 32), (Q8, 96, 16400, 32),   # one (Q8_0 two)
+    (Q4, 11008, 65, 5), (Q6, 11008, 20, 3), (Q8, 11008, 33, 4)])       # the VALU kernel
+def test_matmul_batch_tiles(gpu, oracle_mod, qtype, n, d, tokens):
+    P, O = gpu, oracle_mod
+    print(f"[case] batch type {qtype} n {n} d {d} tokens {tokens}", flush=True)
+    rng = np.random.default_rng([qtype, n, d, tokens])
+    rows = S.random_weights(rng, qtype, n, d, S.unit_scale_exp(qtype, n))
+    W = G.QMatrix(qtype, n, d, rows)
+    X = rng.standard_normal((tokens, n)).astype(np.float32)
+    got = batch(P, W, X)
+    for t in range(tokens):
+        assert_bits(got[t], O.matmul(rows, X[t], n, d, qtype), t)
+    W.free()
+
+
+@pytest.mark.parametrize("qtype", [Q4, Q6, Q8])
+def test_matmul_batch_special_values(gpu, oracle_mod, qtype):
+    """Tokens of subnormal, huge, mixed and zero activations, one with an
+    infinity and one with a NaN (whose rows alone are not finite), and rows
+    with zero scales."""
+    P, O = gpu, oracle_mod
+    n, d, tokens = 512, 40, 24
+    rng = np.random.default_rng(77 + qtype)
+    rows = S.random_weights(rng, qtype, n, d, S.unit_scale_exp(qtype, n))
+    at = {Q4: slice(0, 4), Q6: slice(208, 210), Q8: slice(0, 2)}[qtype]
+    rows.reshape(d, -1, G.BLOCK[qtype][1])[::5, :, at] = 0
+    X = rng.standard_normal((tokens, n)).astype(np.float32)
+    X[1] *= 1e-39
+    X[2] *= 1e-43
+    X[3] *= 1e30
+    X[4] = 0.0
+    X[5] *= np.exp2(rng.integers(-60, 60, n)).astype(np.float32)
+    X[6] = -0.0
+    X[7, 100] = np.inf
+    X[8, 200] = np.nan
+    W = G.QMatrix(qtype, n, d, rows)
+    got = batch(P, W, X)
+    for t in range(tokens):
+        with np.errstate(all="ignore"):
+            want = O.matmul(rows, X[t], n, d, qtype)
+        assert_bits(got[t], want, t)
+    assert np.isfinite(got[[0, 4, 9, 23]]).all() and not np.isfinite(got[7:9]).all()
+    W.free()
