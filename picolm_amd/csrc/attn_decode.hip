@@ -186,6 +186,13 @@ int g_fwd_prefetch = 0;
 int g_fwd_fuse = 0;  // key 17
 int g_xcd_ok[kMaxDevices] = {};
 
+void decode_scratch(unsigned** ctr, float** part, size_t* part_bytes) {
+  char* base = (char*)g_scratch_ptr[ctx().device];
+  *ctr = (unsigned*)base;
+  *part = (float*)(base + kScratchCounterBytes);
+  *part_bytes = kScratchBytes - kScratchCounterBytes;
+}
+
 int decode_scratch_setup(int device) {
   if (device < 0 || device >= kMaxDevices) {
     set_error("plh_init: device %d beyond the %d the static scratch table covers", device,

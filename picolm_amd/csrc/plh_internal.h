@@ -127,6 +127,9 @@ int ensure_workspace(size_t bytes);
 // launch of at most kDecodeCounters / 32 (layer, kv head, q-head block)
 // groups runs it.
 constexpr int kDecodeCounters = 1 << 18;
+// The static scratch of the current device: kDecodeCounters counters (zero
+// between launches) and the partials' region.  Needs no allocation.
+void decode_scratch(unsigned** ctr, float** part, size_t* part_bytes);
 
 // Attention of the head dims without a tuned kernel (every even head_dim up
 // to 256 but 64 and 128; attn_generic.hip): append and attend n_tokens rows

@@ -1,0 +1,172 @@
+"""The generic attention kernels (attn_generic.hip) where their tiles can go
+wrong, against the oracle: every built number of 16-wide d tiles and head dims
+between them (also ones that are not multiples of 4, whose rows are not 8-byte
+aligned), one key to several tiles per wave, key ranges split over workgroups,
+GQA groups that leave partial column tiles or fill several.  Rows after a
+token's own must not reach it whatever they hold; the allocation-free entry
+point and a first call under graph capture work as with the tuned kernels."""
+import numpy as np
+import pytest
+
+import test_gpu_decode as TD
+import test_gpu_prefill as TP
+from attn_check import assert_attn_close, filled_cache, normal_f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [4, 16, 34, 48, 50, 72, 80, 100, 112, 130, 160, 176, 192, 208, 256])
+@pytest.mark.parametrize("pos", [15, 64, 777])
+def test_decode_head_dims(gpu, oracle_mod, D, pos):
+    cfg = gpu.AttnConfig(2, 6, 2, D, 800, 1e4, D // 2 % 2)
+    TD.run_decode(gpu, oracle_mod, cfg, pos, seed=D + pos, poison=True)
+
+
+@pytest.mark.parametrize("heads", [(7, 1), (40, 2), (32, 32), (20, 20)])
+@pytest.mark.parametrize("pos", [16, 63, 1023, 2500])
+def test_decode_groups_and_splits(gpu, oracle_mod, heads, pos):
+    cfg = gpu.AttnConfig(3, heads[0], heads[1], 80, 2600, 1e4, 0)
+    TD.run_decode(gpu, oracle_mod, cfg, pos, seed=pos, check_layers=[1], per_layer=pos == 1023)
+
+
+@pytest.mark.parametrize("case", [  # n_heads, n_kv_heads, head_dim, start, n
+    (4, 4, 20, 0, 16), (4, 4, 48, 0, 17), (14, 2, 80, 5, 33), (8, 2, 96, 700, 3),
+    (6, 6, 112, 64, 65), (8, 8, 144, 0, 40), (2, 1, 176, 31, 50), (2, 2, 250, 0, 70),
+    (8, 8, 80, 1200, 20)])
+def test_prefill_tiles(gpu, oracle_mod, case):
+    Hq, Hkv, D, start, n = case
+    cfg = gpu.AttnConfig(2, Hq, Hkv, D, start + n + 3, 1e4, 1)
+    TP.run_prefill(gpu, oracle_mod, cfg, start, n, seed=D + n)
+
+
+@pytest.mark.parametrize("D,n", [(66, 20), (72, 33), (80, 48), (96, 63), (112, 17), (120, 65)])
+def test_prefill_two_tiles_a_workgroup(gpu, oracle_mod, D, n):
+    """From 4 x 256 column tiles in a launch a workgroup takes two of them:
+    the last one's second tile full, partial or missing."""
+    cfg = gpu.AttnConfig(11, 48, 48, D, n + 2, 1e4, D // 8 % 2)
+    TP.run_prefill(gpu, oracle_mod, cfg, 0, n, seed=D + n, check_layers=[0, 10])
+
+
+def test_decode_unaligned_caches(gpu):
+    """Caches that start 2 elements past a 16-byte boundary (4-byte loads): the
+    same bits as aligned ones."""
+    P = gpu
+    S, D, Hkv, pos = 300, 80, 2, 250
+    rng = np.random.default_rng(5)
+    kc, vc = (normal_f32(rng, (S * Hkv * D,)).astype(np.float16) for _ in "kv")
+    q, k, v = (normal_f32(rng, (h * D,)) for h in (6, Hkv, Hkv))
+    ang = rng.uniform(0, 6, (S, D // 2)).astype(np.float32)
+    d = [P.DeviceBuffer.from_numpy(x) for x in (q, k, v, np.cos(ang), np.sin(ang))]
+    outs = []
+    for off in (0, 2):
+        pad = [np.concatenate([np.zeros(off, np.float16), x]) for x in (kc, vc)]
+        c = [P.DeviceBuffer.from_numpy(x) for x in pad]
+        out = P.DeviceBuffer(4 * 6 * D)
+        P.check(P.lib.plh_attn_decode(1, 6, Hkv, D, S, 0, 0, 1, pos, d[0].ptr, d[1].ptr, d[2].ptr,
+                                      c[0].ptr + 2 * off, c[1].ptr + 2 * off, d[3].ptr, d[4].ptr,
+                                      out.ptr), "plh_attn_decode")
+        P.synchronize()
+        outs.append(out.download(np.uint32, (6 * D,)))
+        row = slice(off + pos * Hkv * D, off + (pos + 1) * Hkv * D)
+        assert np.array_equal(c[1].download(np.float16, pad[1].shape)[row], v.astype(np.float16))
+    assert np.array_equal(outs[0], outs[1])
+
+
+def test_prefill_later_rows_do_not_matter(gpu):
+    """Tokens 0..19 give the same bits whatever finite rows tokens 20..39 hold;
+    with infinities and NaNs among them (whose tiles are taken again in fp32)
+    the same to fp32 rounding: 40 terms of 2^-24 of the largest."""
+    P = gpu
+    cfg = P.AttnConfig(1, 6, 2, 80, 64, 1e4, 0)
+    rng = np.random.default_rng(3)
+    n, outs = 40, []
+    q, k, v = (normal_f32(rng, (n, d)) for d in (cfg.q_dim, cfg.kv_dim, cfg.kv_dim))
+    for bad in (None, 1.0, np.inf, np.nan):
+        if bad is not None:
+            k[20:], v[20:] = normal_f32(rng, k[20:].shape), normal_f32(rng, v[20:].shape)
+            k[21, ::7], v[20:30, ::5] = bad, bad
+        cache = P.KVCache(cfg)
+        d = [P.DeviceBuffer.from_numpy(x) for x in (q, k, v)]
+        out = P.DeviceBuffer(4 * n * cfg.q_dim)
+        P.prefill(cache, 0, 0, n, d[0].ptr, d[1].ptr, d[2].ptr, out.ptr)
+        P.synchronize()
+        outs.append(out.download(np.float32, (n, cfg.q_dim)))
+        cache.free()
+    assert np.isfinite(outs[0]).all()
+    assert np.array_equal(outs[1][:20].view(np.uint32), outs[0][:20].view(np.uint32))
+    for o in outs[2:]:
+        assert np.max(np.abs(o[:20] - outs[0][:20])) <= 40 * 2.0 ** -24 * np.abs(outs[0]).max()
+    assert np.isnan(outs[3][21:]).any()
+
+
+@pytest.mark.parametrize("kind", ["k_inf", "v_inf"])
+def test_decode_infinite_cached_rows(gpu, oracle_mod, kind):
+    """fp16 infinities in the cache (a k or v beyond 65504 rounds to one): a key
+    whose score is minus infinity has no weight, an infinite v reaches its own
+    d alone, as in the reference's fp32 arithmetic."""
+    P, O = gpu, oracle_mod
+    cfg = P.AttnConfig(1, 4, 2, 48, 256, 1e4, 0)
+    pos, rng = 200, np.random.default_rng(11)
+    kc, vc = filled_cache(O, cfg, pos, rng)
+    k3, v3 = kc.reshape(256, 2, 48), vc.reshape(256, 2, 48)
+    q = np.abs(normal_f32(rng, (cfg.q_dim,))) + np.float32(0.1)
+    k, v = normal_f32(rng, (cfg.kv_dim,)), normal_f32(rng, (cfg.kv_dim,))
+    cos_t, sin_t = O.rope_tables(256, 48, 1e4)
+    cos_t[pos], sin_t[pos] = 1.0, 0.0      # no rotation: q stays positive
+    if kind == "k_inf":
+        k3[40, :, 7] = 0xFC00
+    else:
+        v3[40, :, 7] = 0x7C00
+    cache = P.KVCache(cfg)
+    cache.load(kc, vc)
+    cache.cos.upload(cos_t)
+    cache.sin.upload(sin_t)
+    d = [P.DeviceBuffer.from_numpy(x) for x in (q, k, v)]
+    out = P.DeviceBuffer(4 * cfg.q_dim)
+    P.decode(cache, 0, pos, d[0].ptr, d[1].ptr, d[2].ptr, out.ptr)
+    P.synchronize()
+    got = out.download(np.float32, (4, 48))
+    shp = O.Shape(1, 4, 2, 48, 256, 1e4, 0)
+    ref = O.attn_decode(shp, 0, pos, q.copy(), k.copy(), v, kc, vc, cos_t, sin_t).reshape(4, 48)
+    inf = np.zeros(48, bool)
+    inf[7] = kind == "v_inf"
+    assert np.isinf(ref[:, inf]).all() and np.array_equal(got[:, inf], ref[:, inf])
+    assert_attn_close(got[:, ~inf].copy(), ref[:, ~inf].copy(), 48 - inf.sum(), what=kind)
+    cache.free()
+
+
+def test_decode_capture_and_noalloc(gpu, oracle_mod):
+    """A split launch captured at its first call and replayed, and the
+    allocation-free entry point: the eager call's bits each time."""
+    P, O = gpu, oracle_mod
+    cfg = P.AttnConfig(2, 8, 4, 96, 1100, 1e4, 0)
+    pos, rng = 1000, np.random.default_rng(9)
+    kc, vc = filled_cache(O, cfg, pos, rng)
+    q, k, v = (normal_f32(rng, (2, d)) for d in (cfg.q_dim, cfg.kv_dim, cfg.kv_dim))
+    d = [P.DeviceBuffer.from_numpy(x) for x in (q, k, v)]
+    outs = [P.DeviceBuffer(4 * 2 * cfg.q_dim) for _ in range(3)]
+    caches = [P.KVCache(cfg) for _ in range(3)]
+    for c in caches:
+        c.load(kc, vc)
+    with P.Graph() as gr:
+        P.decode(caches[0], 0, pos, d[0].ptr, d[1].ptr, d[2].ptr, outs[0].ptr, 2)
+    P.decode(caches[1], 0, pos, d[0].ptr, d[1].ptr, d[2].ptr, outs[1].ptr, 2)
+    P.synchronize()
+    eager = outs[1].download(np.float32, (2, cfg.q_dim))
+    c = caches[2]
+    P.check(P.lib.plh_attn_decode_noalloc(2, 8, 4, 96, 1100, 0, 0, 2, pos, d[0].ptr, d[1].ptr,
+                                          d[2].ptr, c.key.ptr, c.val.ptr, c.cos.ptr, c.sin.ptr,
+                                          outs[2].ptr), "plh_attn_decode_noalloc")
+    P.synchronize()
+    assert np.array_equal(outs[2].download(np.float32, eager.shape), eager)
+    for _ in range(3):
+        outs[0].zero()
+        gr.launch()
+        P.synchronize()
+        assert np.array_equal(outs[0].download(np.float32, eager.shape), eager)
+        P.decode(caches[1], 0, pos, d[0].ptr, d[1].ptr, d[2].ptr, outs[1].ptr, 2)
+        P.synchronize()
+    shp = O.Shape(2, 8, 4, 96, 1100, 1e4, 0)
+    cos_t, sin_t = O.rope_tables(1100, 96, 1e4)
+    ref = O.attn_decode(shp, 1, pos, q[1].copy(), k[1].copy(), v[1], kc, vc, cos_t, sin_t)
+    assert_attn_close(eager[1], ref, 96, what="layer 1")
