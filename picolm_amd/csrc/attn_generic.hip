@@ -1,5 +1,6 @@
 // attn_generic.hip -- decode and prefill attention for head dims without a
-// tuned kernel (every even head_dim up to 256 but 64 and 128).
+// tuned kernel (every even head_dim up to 256 but 64 and 128), and small
+// prefill launches of these two (few_tiles_pay, attn_prefill.hip).
 //
 // Replaces the same reference code as the tuned kernels: model.c:807-892
 // (decode: QK-norm, RoPE, fp16 append at row pos, online-softmax GQA
@@ -275,12 +276,15 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
                "s"(a.fd_split.m), "s"(a.fd_split.sh), "s"(a.fd_tiles.m));
   const int D = a.D, kv_dim = a.n_kv_heads * D;
   const int G = (int)fdiv(a.n_heads, a.fd_kvh);
-  // unit -> (group, split); group -> (layer, kv head, column tile), the tiles
-  // with the most keys first
-  const int group = (int)fdiv(blockIdx.x, a.fd_split), split = blockIdx.x - group * a.n_split;
-  const int gt = (int)fdiv(group, a.fd_tiles);
-  const int tile = a.col_tiles - 1 - (group - gt * a.col_tiles);
-  const int li = (int)fdiv(gt, a.fd_kvh), kvh = gt - li * a.n_kv_heads;
+  // workgroup -> kv head, split, column tile (the tiles with the most keys
+  // first), layer.  Workgroup b runs on XCD b % 8: with 8 kv heads or a multiple
+  // an XCD's L2 holds its own heads' rows only (300 tokens, head_dim 80, 32 heads:
+  // 23.1 us with the column tile fastest, 19.2 so).
+  const int bh = (int)fdiv(blockIdx.x, a.fd_kvh), kvh = blockIdx.x - bh * a.n_kv_heads;
+  const int bs = (int)fdiv(bh, a.fd_split), split = bh - bs * a.n_split;
+  const int li = (int)fdiv(bs, a.fd_tiles);
+  const int tile = a.col_tiles - 1 - (bs - li * a.col_tiles);
+  const int group = bs * a.n_kv_heads + kvh;
   const int cols = a.n_tokens * G;
   const int w0 = NC * tile;                                   // the workgroup's first column
   const int c0 = min(w0 + 16 * cw, cols - 1);                 // this wave's
@@ -579,7 +583,7 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
         if (d + i < D) ot[i] = O[i] * inv;
     } else {  // KS 4: one column tile
       const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-          a.part + (size_t)blockIdx.x * Sh::kPart, 0, Sh::kPart * 4, 0x00020000);
+          a.part + ((size_t)group * a.n_split + split) * Sh::kPart, 0, Sh::kPart * 4, 0x00020000);
       __builtin_amdgcn_raw_buffer_store_b128(O, prs, (col * Sh::DP + d) * 4, 0, kDeviceScope);
       if (d == 0) {
         const int at = (16 * Sh::DP + 2 * col) * 4;
@@ -694,7 +698,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
                  const float* k, const float* v, uint16_t* key_cache, uint16_t* val_cache,
                  const float* rope_cos, const float* rope_sin, float* out, int out_stride,
                  const float* q_norm, const float* k_norm, float norm_eps, uint16_t* k_rows,
-                 uint16_t* v_rows) {
+                 uint16_t* v_rows, bool append) {
   if (head_dim < 2 || head_dim > kGMaxD || head_dim % 2) {
     set_error("attention: head_dim %d must be even and at most %d", head_dim, kGMaxD);
     return -1;
@@ -714,7 +718,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // 512 workgroups: 15.5 / 11.3 / 13.5 / 12.6), as far as every wave keeps a
   // tile, the partials fit the static scratch and the merges its counters.
   const int G = n_heads / n_kv_heads, cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  a.fuse = n_tokens == 1;
+  a.fuse = append && n_tokens == 1;
   const int dt = built_tiles(head_dim), kmax = start_pos + n_tokens;
   const long tiles = (long)n_kv_heads * ((n_tokens * G + 15) / 16) * n_launch_layers;
   // Two column tiles a workgroup halve its fixed chain per column but give a
@@ -776,7 +780,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
     if (k_rows) b.k_rows = k_rows + rows_before * kv_dim;
     if (v_rows) b.v_rows = v_rows + rows_before * kv_dim;
     const long nl = b.n_launch_layers;
-    if (!a.fuse) {
+    if (append && !a.fuse) {
       const long rows = nl * n_tokens * n_kv_heads;
       if (b.kn)
         hipLaunchKernelGGL(generic_append_norm_kernel, dim3((unsigned)rows), dim3(kGThreads), 0,

@@ -785,6 +785,31 @@ int g_prefill_split = 0;
 int g_prefill_ksplit = 0;
 }  // namespace plh
 
+// Whether a launch runs on the generic kernel's 16-column tiles (after the
+// append kernel here; a single token's row is appended in its own launch).
+// They give a launch of few units eight times the workgroups, each wave a share
+// of the keys, and need no merge launch; a 32-column wave does more products
+// per K/V byte and LDS read once every CU has work.  One-layer launches with
+// their append, units -> tiles, us: 128 tokens at head_dim 64, 32 q and 4 kv
+// heads 11.5 -> 9.1, at start 1000 22.6 -> 17.0; 509 tokens at head_dim 128, 16
+// q and 8 kv heads 28.7 -> 24.7; one token after 8000 38 -> 17.  Launches of
+// more units than a quarter of the CUs lose (512 tokens of the first: 18.0 ->
+// 21.1), and so do long contexts, by wave tiles (32 keys, 16 columns) per CU:
+// above about 50 at head_dim 64 (128 tokens at start 8000: 55 -> 67 us) and 20
+// at 128 (200 tokens at start 1000: 29 -> 33), unless the unit's columns fill
+// one wave in four at most (2 tokens at start 8000, 22 layers: 125 -> 49).
+// Prompts within two key tiles take either way the same time.
+static bool few_tiles_pay(const PrefillArgs& a, int head_dim, int cus) {
+  if (g_prefill_split || g_prefill_ksplit) return false;  // the units' own splits, by tuning
+  const long G = a.n_heads / a.n_kv_heads, cols = a.n_tokens * G;
+  const long key_tiles = (a.start_pos + a.n_tokens + kKT - 1) / kKT;
+  if (a.n_tokens == 1 || (cols <= 32 && key_tiles > 8)) return true;
+  const double tiles = (double)a.n_launch_layers * a.n_kv_heads * ((cols + 15) / 16) *
+                       (a.start_pos + 0.5 * a.n_tokens) / kKT;
+  return (long)a.n_units * 4 <= cus && key_tiles >= 3 &&
+         tiles <= (head_dim == 64 ? 48.0 : 20.0) * cus;
+}
+
 static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head_dim,
                              int max_seq_len, int rope_type, int layer0, int n_launch_layers,
                              int start_pos, int n_tokens, const float* q, const float* k,
@@ -876,6 +901,14 @@ static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head
   const long slots = 3L * (c.num_cus > 0 ? c.num_cus : 256);
   a.paired = a.n_qblk >= 4 && a.n_units >= 8 * slots ? 1 : 0;
   a.per_xcd = a.groups_per_xcd * (a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk);
+  const bool few = few_tiles_pay(a, head_dim, c.num_cus > 0 ? c.num_cus : 256);
+  auto small = [&](bool append) {
+    return attn_generic(n_heads, n_kv_heads, head_dim, max_seq_len, rope_type, layer0,
+                        n_launch_layers, start_pos, n_tokens, q, k, v, key_cache, val_cache,
+                        rope_cos, rope_sin, out, out_stride, q_norm, k_norm, norm_eps, nullptr,
+                        nullptr, append);
+  };
+  if (few && n_tokens == 1) return small(true);
   // Launches with few q blocks (one layer of a prompt chunk, or of a short
   // or narrow prompt: at most a quarter as many blocks as CUs) split their
   // blocks into chunks of T tiles, merged afterwards: the heaviest block is
@@ -886,7 +919,7 @@ static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head
   // launches with more blocks lose to the extra prologues and the merge.
   a.split_tiles = 0;
   a.chunks_per_group = 0;
-  if (!a.paired && g_prefill_split >= 0) {
+  if (!few && !a.paired && g_prefill_split >= 0) {
     const int max_tiles = prefill_unit_tiles(a, a.n_qblk - 1);
     const int cus = c.num_cus > 0 ? c.num_cus : 256;
     auto chunks_of = [&](int T) {
@@ -962,6 +995,7 @@ static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head
       hipLaunchKernelGGL((prefill_append_kernel<128, false>), ag, ab256, 0, c.stream, a);
   }
   if (check_hip(hipGetLastError(), "prefill_append_kernel")) return -1;
+  if (few) return small(false);
   if (ksplit > 0) {
     const dim3 kg((unsigned)a.n_units), kb((unsigned)(kPThreads * ksplit));
     if (head_dim == 64 && ksplit == 3) {

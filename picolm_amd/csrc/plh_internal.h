@@ -131,16 +131,16 @@ constexpr int kDecodeCounters = 1 << 18;
 // between launches) and the partials' region.  Needs no allocation.
 void decode_scratch(unsigned** ctr, float** part, size_t* part_bytes);
 
-// Attention of the head dims without a tuned kernel (every even head_dim up
-// to 256 but 64 and 128; attn_generic.hip): append and attend n_tokens rows
-// at start_pos.. of layers layer0.. (decode: n_tokens 1, out_stride
-// n_heads*head_dim).  Arguments are checked by the caller.  0 or -1.
+// Attention on 16-column tiles (attn_generic.hip): every even head_dim up to
+// 256.  Appends, unless the rows are there already (append false), and attends
+// n_tokens rows at start_pos.. of layers layer0.. (decode: n_tokens 1,
+// out_stride n_heads*head_dim).  Arguments are checked by the caller.  0 or -1.
 int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int rope_type,
                  int layer0, int n_launch_layers, int start_pos, int n_tokens, const float* q,
                  const float* k, const float* v, uint16_t* key_cache, uint16_t* val_cache,
                  const float* rope_cos, const float* rope_sin, float* out, int out_stride,
                  const float* q_norm, const float* k_norm, float norm_eps, uint16_t* k_rows,
-                 uint16_t* v_rows);
+                 uint16_t* v_rows, bool append = true);
 
 // Decode kernel arguments (all device pointers).
 struct DecodeArgs {

@@ -72,6 +72,50 @@ def test_decode_unaligned_caches(gpu):
     assert np.array_equal(outs[0], outs[1])
 
 
+FEW = [  # n_layers, n_heads, n_kv_heads, head_dim, rope_type, qk_norm, start, n, stride pad
+    (3, 32, 4, 64, 0, False, 0, 1, 0), (2, 8, 4, 128, 1, True, 900, 1, 4),
+    (1, 14, 2, 64, 0, True, 300, 1, 0), (1, 32, 4, 64, 1, False, 0, 65, 4),
+    (1, 14, 2, 64, 1, True, 200, 100, 0), (1, 16, 8, 128, 1, True, 0, 509, 0),
+    (1, 28, 4, 128, 0, False, 17, 80, 8), (22, 12, 4, 64, 0, False, 260, 10, 0),
+    (9, 16, 8, 128, 1, True, 400, 16, 0), (1, 128, 1, 64, 0, False, 90, 6, 0)]
+
+
+@pytest.mark.parametrize("case", FEW)
+def test_small_prefill_launches_match_units(gpu, case):
+    """Head dims 64 and 128: the 16-column tiles of small launches against the
+    32-column units (plh_set_tuning key 5 at -1) on the same inputs.  The same
+    appended rows bit for bit, outputs within the units' hi/lo precision."""
+    L, Hq, Hkv, D, rope, norm, start, n, pad = case
+    P = gpu
+    cfg = P.AttnConfig(L, Hq, Hkv, D, start + n + 1, 1e4, rope)
+    rng = np.random.default_rng(start + n)
+    rows = cfg.max_seq_len * L * cfg.kv_dim
+    kc, vc = (normal_f32(rng, (rows,)).astype(np.float16).view(np.uint16) for _ in "kv")
+    ins = [normal_f32(rng, (L, n, w)) for w in (cfg.q_dim, cfg.kv_dim, cfg.kv_dim)]
+    ins += [rng.uniform(0.5, 1.5, (L, D)).astype(np.float32) for _ in "qk"]
+    d = [P.DeviceBuffer.from_numpy(x) for x in ins]
+    kw = dict(q_norm=d[3].ptr, k_norm=d[4].ptr, norm_eps=1e-5) if norm else {}
+    got = []
+    for key5 in (0, -1):
+        cache = P.KVCache(cfg)
+        cache.load(kc, vc)
+        out = P.DeviceBuffer(4 * L * n * (cfg.q_dim + pad))
+        out.zero()
+        P.check(P.lib.plh_set_tuning(5, key5), "plh_set_tuning")
+        try:
+            P.prefill(cache, 0, start, n, d[0].ptr, d[1].ptr, d[2].ptr, out.ptr,
+                      cfg.q_dim + pad, L, **kw)
+            P.synchronize()
+        finally:
+            P.lib.plh_set_tuning(5, 0)
+        got.append((out.download(np.float32, (L * n, cfg.q_dim + pad)), *cache.fetch()))
+        cache.free()
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(a, b)
+    assert not got[0][0][:, cfg.q_dim:].any()
+    assert_attn_close(got[0][0][:, :cfg.q_dim], got[1][0][:, :cfg.q_dim], D, what="few")
+
+
 def test_prefill_later_rows_do_not_matter(gpu):
     """Tokens 0..19 give the same bits whatever finite rows tokens 20..39 hold;
     with infinities and NaNs among them (whose tiles are taken again in fp32)
