@@ -810,13 +810,12 @@ static bool few_tiles_pay(const PrefillArgs& a, int head_dim, int cus) {
          tiles <= (head_dim == 64 ? 48.0 : 20.0) * cus;
 }
 
-static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head_dim,
-                             int max_seq_len, int rope_type, int layer0, int n_launch_layers,
-                             int start_pos, int n_tokens, const float* q, const float* k,
-                             const float* v, uint16_t* key_cache, uint16_t* val_cache,
-                             const float* rope_cos, const float* rope_sin, float* out,
-                             int out_stride, const float* q_norm, const float* k_norm,
-                             float norm_eps) {
+int plh::attn_prefill(int n_layers, int n_heads, int n_kv_heads, int head_dim, int max_seq_len,
+                      int rope_type, int layer0, int n_launch_layers, int start_pos, int n_tokens,
+                      const float* q, const float* k, const float* v, uint16_t* key_cache,
+                      uint16_t* val_cache, const float* rope_cos, const float* rope_sin,
+                      float* out, int out_stride, const float* q_norm, const float* k_norm,
+                      float norm_eps, bool small) {
   Context& c = ctx();
   if (!c.stream) {
     set_error("plh_attn_prefill: library not initialised");
@@ -901,14 +900,14 @@ static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head
   const long slots = 3L * (c.num_cus > 0 ? c.num_cus : 256);
   a.paired = a.n_qblk >= 4 && a.n_units >= 8 * slots ? 1 : 0;
   a.per_xcd = a.groups_per_xcd * (a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk);
-  const bool few = few_tiles_pay(a, head_dim, c.num_cus > 0 ? c.num_cus : 256);
-  auto small = [&](bool append) {
+  const bool few = small && few_tiles_pay(a, head_dim, c.num_cus > 0 ? c.num_cus : 256);
+  auto tiles = [&](bool append) {
     return attn_generic(n_heads, n_kv_heads, head_dim, max_seq_len, rope_type, layer0,
                         n_launch_layers, start_pos, n_tokens, q, k, v, key_cache, val_cache,
                         rope_cos, rope_sin, out, out_stride, q_norm, k_norm, norm_eps, nullptr,
                         nullptr, append);
   };
-  if (few && n_tokens == 1) return small(true);
+  if (few && n_tokens == 1) return tiles(true);
   // Launches with few q blocks (one layer of a prompt chunk, or of a short
   // or narrow prompt: at most a quarter as many blocks as CUs) split their
   // blocks into chunks of T tiles, merged afterwards: the heaviest block is
@@ -995,7 +994,7 @@ static int attn_prefill_impl(int n_layers, int n_heads, int n_kv_heads, int head
       hipLaunchKernelGGL((prefill_append_kernel<128, false>), ag, ab256, 0, c.stream, a);
   }
   if (check_hip(hipGetLastError(), "prefill_append_kernel")) return -1;
-  if (few) return small(false);
+  if (few) return tiles(false);
   if (ksplit > 0) {
     const dim3 kg((unsigned)a.n_units), kb((unsigned)(kPThreads * ksplit));
     if (head_dim == 64 && ksplit == 3) {
@@ -1045,9 +1044,9 @@ extern "C" int plh_attn_prefill(int n_layers, int n_heads, int n_kv_heads, int h
                                 const float* v, uint16_t* key_cache, uint16_t* val_cache,
                                 const float* rope_cos, const float* rope_sin, float* out,
                                 int out_stride) {
-  return attn_prefill_impl(n_layers, n_heads, n_kv_heads, head_dim, max_seq_len, rope_type,
-                           layer0, n_launch_layers, start_pos, n_tokens, q, k, v, key_cache,
-                           val_cache, rope_cos, rope_sin, out, out_stride, nullptr, nullptr, 0.0f);
+  return attn_prefill(n_layers, n_heads, n_kv_heads, head_dim, max_seq_len, rope_type, layer0,
+                      n_launch_layers, start_pos, n_tokens, q, k, v, key_cache, val_cache,
+                      rope_cos, rope_sin, out, out_stride, nullptr, nullptr, 0.0f, true);
 }
 
 extern "C" int plh_attn_prefill_qknorm(int n_layers, int n_heads, int n_kv_heads, int head_dim,
@@ -1058,8 +1057,7 @@ extern "C" int plh_attn_prefill_qknorm(int n_layers, int n_heads, int n_kv_heads
                                        const float* rope_cos, const float* rope_sin, float* out,
                                        int out_stride, const float* q_norm, const float* k_norm,
                                        float norm_eps) {
-  return attn_prefill_impl(n_layers, n_heads, n_kv_heads, head_dim, max_seq_len, rope_type,
-                           layer0, n_launch_layers, start_pos, n_tokens, q, k, v, key_cache,
-                           val_cache, rope_cos, rope_sin, out, out_stride, q_norm, k_norm,
-                           norm_eps);
+  return attn_prefill(n_layers, n_heads, n_kv_heads, head_dim, max_seq_len, rope_type, layer0,
+                      n_launch_layers, start_pos, n_tokens, q, k, v, key_cache, val_cache,
+                      rope_cos, rope_sin, out, out_stride, q_norm, k_norm, norm_eps, true);
 }

@@ -472,17 +472,15 @@ int prefill_chunk(const plh_model* m, const int* tokens, int T, int pos0, const 
                              call(L.v, E, KV, a.xn, E, a.v, KV, L.v_bias, nullptr, nullptr)};
     if (launch_rmsnorm_rows(a.x, L.attn_norm, a.xn, E, T, eps) || gemv_batch3_launch(qkv))
       return -1;
-    // model.c:1019-1090: QK-norm, RoPE, fp16 append and attention per token
-    const int rc =
-        L.q_norm ? plh_attn_prefill_qknorm(m->n_layers, m->n_heads, m->n_kv_heads, m->head_dim,
-                                           m->max_seq_len, m->rope_type, l, 1, pos0, T, a.q, a.k,
-                                           a.v, m->key_cache, m->val_cache, m->rope_cos,
-                                           m->rope_sin, a.att, Q, L.q_norm, L.k_norm, eps)
-                 : plh_attn_prefill(m->n_layers, m->n_heads, m->n_kv_heads, m->head_dim,
-                                    m->max_seq_len, m->rope_type, l, 1, pos0, T, a.q, a.k, a.v,
-                                    m->key_cache, m->val_cache, m->rope_cos, m->rope_sin, a.att,
-                                    Q);
-    if (rc) return -1;
+    // model.c:1019-1090: QK-norm, RoPE, fp16 append and attention per token.
+    // Not on the small launches' tiles: 4 us of a layer's 240, and a prompt
+    // keeps its bits (a score's last bit moves cached fp16 values of later
+    // layers, and these the logits by 1e-3).
+    if (attn_prefill(m->n_layers, m->n_heads, m->n_kv_heads, m->head_dim, m->max_seq_len,
+                     m->rope_type, l, 1, pos0, T, a.q, a.k, a.v, m->key_cache, m->val_cache,
+                     m->rope_cos, m->rope_sin, a.att, Q, L.q_norm,
+                     L.q_norm ? L.k_norm : nullptr, eps, false))
+      return -1;
     // model.c:1092-1107: output projection, its bias where present, residual
     if (gemv_launch(call(L.o, Q, E, a.att, Q, a.x, E, L.o_bias, nullptr, a.x))) return -1;
     // model.c:1109-1139: rmsnorm, gate / up, silu * up, down, residual

@@ -131,6 +131,14 @@ constexpr int kDecodeCounters = 1 << 18;
 // between launches) and the partials' region.  Needs no allocation.
 void decode_scratch(unsigned** ctr, float** part, size_t* part_bytes);
 
+// plh_attn_prefill(_qknorm; q_norm and k_norm null without).  small: a launch
+// of head_dim 64 or 128 may take the 16-column tiles (few_tiles_pay).
+int attn_prefill(int n_layers, int n_heads, int n_kv_heads, int head_dim, int max_seq_len,
+                 int rope_type, int layer0, int n_launch_layers, int start_pos, int n_tokens,
+                 const float* q, const float* k, const float* v, uint16_t* key_cache,
+                 uint16_t* val_cache, const float* rope_cos, const float* rope_sin, float* out,
+                 int out_stride, const float* q_norm, const float* k_norm, float norm_eps,
+                 bool small);
 // Attention on 16-column tiles (attn_generic.hip): every even head_dim up to
 // 256.  Appends, unless the rows are there already (append false), and attends
 // n_tokens rows at start_pos.. of layers layer0.. (decode: n_tokens 1,
