@@ -21,8 +21,8 @@
 // MFMA cycles + ~150 x 4 VALU cycles (88 of them the exact order's own adds
 // and products).  TinyLlama's 128-token prompt, us a launch before (the VALU
 // kernel) and now: gate/up pair (5632 x 2048 Q4_K twice) 340 -> 96, down (2048 x
-// 5632 Q6_K) 287 -> 75, o 70 -> 25, q, k and v 102 in three launches -> 31 in
-// one; the whole prompt 18.1 -> 5.8 ms.  Set aside: x straight from the caches
+// 5632 Q6_K) 287 -> 77, o 70 -> 25, q, k and v 102 in three launches -> 36 in
+// one; the whole prompt 18.1 -> 5.5 ms.  Set aside: x straight from the caches
 // instead of LDS (Q4_K 11264 x 2048, 128 tokens: 136 us against 96, Q6_K 387
 // against 130: the vector memory path handles the 16 tokens' lines one by
 // one); two token tiles a wave (88 against 94 us on that shape, slower below it).
@@ -508,9 +508,10 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemvArgs a, BatchSh
     gemm_body<F, KW, PAIR>(a, b, r_tile, t_tile, lds);
 }
 
-// Up to three matrices over the same x in one launch (q, k and v), the row
-// tiles of each a range of the grid's: a small matrix alone leaves most CUs
-// idle.
+// Three matrices over the same x in one launch (q, k and v), the row tiles of
+// each a range of the grid's: a small matrix alone leaves most CUs idle.  K
+// quants and Q8_0 are built apart: with both, Q8_0's registers leave two
+// workgroups a CU instead of three.
 struct MultiBatch {
   GemvArgs seg[3];
   BatchShape shape[3];  // row_tiles: of the segment
@@ -518,21 +519,19 @@ struct MultiBatch {
   int tile1, tile2, row_tiles;  // first tiles of segments 1 and 2, all tiles
 };
 
-template <int KW>
+template <int KW, bool Q8>
 __global__ __launch_bounds__(kThreads) void gemm_mfma_multi_kernel(MultiBatch m) {
   extern __shared__ __align__(16) float lds[];
   int r_tile, t_tile;
   if (!tile_of(m.row_tiles, m.shape[0].tok_tiles, r_tile, t_tile)) return;
   const int i = (r_tile >= m.tile1) + (r_tile >= m.tile2);
   r_tile -= i == 2 ? m.tile2 : i == 1 ? m.tile1 : 0;
-  switch (m.qtype[i]) {
-    case kTypeQ4K: gemm_body<Q4KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds); break;
-    case kTypeQ8_0:  // never with KW 1 (waves_per_tile)
-      if constexpr (KW > 1)
-        gemm_body<Q80M, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
-      break;
-    default: gemm_body<Q6KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds); break;
-  }
+  if constexpr (Q8)
+    gemm_body<Q80M, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
+  else if (m.qtype[i] == kTypeQ4K)
+    gemm_body<Q4KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
+  else
+    gemm_body<Q6KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
 }
 
 int cu_count() { return ctx().num_cus > 0 ? ctx().num_cus : 256; }
@@ -588,12 +587,12 @@ void launch_f(int kw, bool pair, const GemvArgs& a, const BatchShape& b, hipStre
   }
 }
 
-template <int KW>
+template <int KW, bool Q8>
 void launch_multi(const MultiBatch& m, hipStream_t st) {
-  size_t lds = std::max(lds_bytes<Q4KM, KW, false>(), lds_bytes<Q6KM, KW, false>());
-  if constexpr (KW > 1) lds = std::max(lds, lds_bytes<Q80M, KW, false>());
-  hipLaunchKernelGGL((gemm_mfma_multi_kernel<KW>), dim3(grid_of(m.row_tiles, m.shape[0].tok_tiles)),
-                     dim3(kThreads), lds, st, m);
+  const size_t lds = Q8 ? lds_bytes<Q80M, KW, false>()
+                        : std::max(lds_bytes<Q4KM, KW, false>(), lds_bytes<Q6KM, KW, false>());
+  hipLaunchKernelGGL((gemm_mfma_multi_kernel<KW, Q8>),
+                     dim3(grid_of(m.row_tiles, m.shape[0].tok_tiles)), dim3(kThreads), lds, st, m);
 }
 
 }  // namespace
@@ -629,15 +628,17 @@ int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, 
   return check_hip(hipGetLastError(), "gemm_mfma_kernel launch");
 }
 
+bool gemm_mfma_multi_takes(const int* qtype) {
+  const int q8 = (qtype[0] == kTypeQ8_0) + (qtype[1] == kTypeQ8_0) + (qtype[2] == kTypeQ8_0);
+  return q8 == 0 || q8 == 3;
+}
+
 int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride,
                     const int* out_stride) {
   MultiBatch m{};
   long tiles = 0;
-  bool q8 = false;
-  for (int i = 0; i < 3; ++i) {
-    tiles += tiles_of(a[i], n_tok);
-    q8 = q8 || qtype[i] == kTypeQ8_0;
-  }
+  for (int i = 0; i < 3; ++i) tiles += tiles_of(a[i], n_tok);
+  const bool q8 = qtype[0] == kTypeQ8_0;
   const int kw = waves_per_tile(tiles, q8);
   for (int i = 0; i < 3; ++i) {
     m.seg[i] = a[i];
@@ -647,12 +648,19 @@ int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride
   m.tile1 = m.shape[0].row_tiles;
   m.tile2 = m.tile1 + m.shape[1].row_tiles;
   m.row_tiles = m.tile2 + m.shape[2].row_tiles;
-  if (kw == 1)
-    launch_multi<1>(m, ctx().stream);
-  else if (kw == 2)
-    launch_multi<2>(m, ctx().stream);
-  else
-    launch_multi<4>(m, ctx().stream);
+  hipStream_t st = ctx().stream;
+  if (q8) {  // never with one wave (waves_per_tile)
+    if (kw == 2)
+      launch_multi<2, true>(m, st);
+    else
+      launch_multi<4, true>(m, st);
+  } else if (kw == 1) {
+    launch_multi<1, false>(m, st);
+  } else if (kw == 2) {
+    launch_multi<2, false>(m, st);
+  } else {
+    launch_multi<4, false>(m, st);
+  }
   return check_hip(hipGetLastError(), "gemm_mfma_multi_kernel launch");
 }
 

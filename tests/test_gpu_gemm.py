@@ -83,3 +83,38 @@ def test_matmul_batch_special_values(gpu, oracle_mod, qtype):
         assert_bits(got[t], want, t)
     assert np.isfinite(got[[0, 4, 9, 23]]).all() and not np.isfinite(got[7:9]).all()
     W.free()
+
+
+def layer0_rows_exact(P, O, n_tok, **kw):
+    """A prompt's layer-0 cached rows (exact order, nothing transcendental)
+    against the oracle's, bit for bit."""
+    cfg = dict(n_layers=1, n_ffn=256, n_heads=4, n_kv_heads=2, head_dim=64, vocab_size=64,
+               max_seq_len=n_tok + 3, rope_type=0, rope_base=1e4, eps=1e-5, **kw)
+    h = S.SynthModel(**cfg, seed=cfg["n_embd"])
+    dm, orc = P.DeviceModel(h), O.OracleForward(h)
+    toks = np.arange(n_tok, dtype=np.int32) % 64
+    try:
+        dm.prefill(toks, 1)
+        P.synchronize()
+        orc.prefill(toks, 1, n_threads=8)
+        for a, b in zip(dm.fetch_cache(), (orc.kc, orc.vc)):
+            assert np.array_equal(a, b)
+    finally:
+        dm.free()
+
+
+@pytest.mark.parametrize("n_embd", [96, 544, 4096, 4128, 8448, 12288])
+def test_prompt_norm_rows(gpu, oracle_mod, n_embd):
+    """rmsnorm rows from short of one piece a thread to several batches of
+    registers."""
+    kinds = ("embd", "output", "q", "k", "v", "o", "gate", "up", "down")
+    layer0_rows_exact(gpu, oracle_mod, 5, n_embd=n_embd, types={k: Q8 for k in kinds})
+
+
+@pytest.mark.parametrize("q,k,v", [(Q4, Q4, Q6), (Q6, Q6, Q4), (Q8, Q8, Q8), (Q4, Q8, Q6),
+                                   (Q8, Q4, Q4)])
+@pytest.mark.parametrize("n_tok", [17, 120])
+def test_prompt_qkv_launches(gpu, oracle_mod, q, k, v, n_tok):
+    """q, k and v of a prompt: K quants or Q8_0 in one launch, mixed in three."""
+    types = dict(embd=Q8, output=Q8, q=q, k=k, v=v, o=Q4, gate=Q4, up=Q4, down=Q4)
+    layer0_rows_exact(gpu, oracle_mod, n_tok, n_embd=768, types=types)
