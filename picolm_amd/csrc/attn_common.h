@@ -293,7 +293,9 @@ __host__ __device__ inline int rms_sq_pitch(int n) { return (n / 8 + 3) / 4 * 4 
 
 // The eight chains and the fold, once every square x[8i+j]^2 of the vector
 // sits at sq[j * pitch + i] (see rms_scale_block).
-template <int NT>
+// AHEAD: the next 32 squares of a chain are read while these are added (32 more
+// registers).
+template <int NT, bool AHEAD = false>
 __device__ __forceinline__ float rms_chain_fold(const float* x, int n, float eps, const float* sq,
                                                 float* red) {
   const int tid = threadIdx.x;
@@ -303,10 +305,18 @@ __device__ __forceinline__ float rms_chain_fold(const float* x, int n, float eps
     const float* s = sq + tid * pitch;
     float acc = 0.0f;
     int i = 0;
-    for (; i + 32 <= n8; i += 32) {
-      float4 v[8];
+    float4 v[8], next[8];
+    if (AHEAD && n8 >= 32) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = *(const float4*)(s + i + 4 * k);
+      for (int k = 0; k < 8; ++k) next[k] = *(const float4*)(s + 4 * k);
+    }
+    for (; i + 32 <= n8; i += 32) {
+      const int at = AHEAD ? min(i + 32, n8 / 32 * 32 - 32) : i;  // the last ones: again
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (AHEAD) v[k] = next[k];
+        (AHEAD ? next : v)[k] = *(const float4*)(s + at + 4 * k);
+      }
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         acc = acc + v[k].x;
