@@ -39,13 +39,15 @@ namespace {
 constexpr int kMT = 16;         // tokens and rows of one MFMA tile
 constexpr int kSubPitch = 36;   // staged floats per 32 elements of x (4 of padding)
 
-// x is staged in chunks: 256 elements, or 128 where the exchanged terms (KW 2)
-// would otherwise take the LDS of a second workgroup.  Staged floats per
+// x is staged in chunks: a unit per wave of 8 (512 elements), else 256, or 128
+// where the exchanged terms (KW 2) would otherwise take the LDS of a second
+// workgroup.  Staged floats per
 // token: a pitch of 4 mod 16 floats, so that 16 tokens' 16-byte reads hit
 // different banks.
+constexpr int waves_of(int kw) { return kw == 8 ? 8 : 4; }  // of a workgroup
 template <int KW>
 struct Chunk {
-  static constexpr int K = KW == 2 ? 128 : 256, U = K / 64;
+  static constexpr int K = KW == 8 ? 512 : KW == 2 ? 128 : 256, U = K / 64;
   static constexpr int kTokPitch = K / 32 * kSubPitch + 4;
   static constexpr int kXs = kMT * kTokPitch;   // floats of a buffer
   static constexpr int kSums = K / 32 * kMT;    // its sub-block sums [sub][token]
@@ -323,25 +325,25 @@ constexpr int x_floats() {
 }
 template <class F, int KW, int M>
 constexpr int term_floats() {
-  return KW == 1 ? 0 : 4 / KW * Chunk<KW>::U * F::kUnitTerms * M * 4 * 64;
+  return KW == 1 ? 0 : waves_of(KW) / KW * Chunk<KW>::U * F::kUnitTerms * M * 4 * 64;
 }
 template <class F, int KW, bool PAIR>
 constexpr size_t lds_bytes() {
   return sizeof(float) * 2 * (size_t)(x_floats<F, KW>() + term_floats<F, KW, PAIR ? 2 : 1>());
 }
 
-// One workgroup: 16 tokens x (4 / KW) * 16 rows (of two matrices for a gate/up
-// pair).  The four waves take row tiles of their own (KW 1), or KW waves share
-// a row tile: each forms the terms of a KW-th of a chunk's units into LDS,
-// then chains a KW-th of the tile's sums over the chunk's terms, in block
-// order.  One barrier per chunk; the next chunk's x, the next unit's operand
+// One workgroup: 16 tokens x (4 / KW) * 16 rows (16 with KW 8; of two matrices
+// for a gate/up pair).  The waves take row tiles of their own (KW 1), or KW
+// waves share a row tile: each forms the terms of a KW-th of a chunk's units
+// into LDS, then chains a KW-th of the tile's sums (KW 8: the first four waves a
+// quarter) over the chunk's terms, in block order.  One barrier per chunk; the next chunk's x, the next unit's operand
 // and the weights of the next two units are in flight meanwhile.
 template <class F, int KW, bool PAIR>
 __device__ __forceinline__ void gemm_body(const GemvArgs& a, const BatchShape& b, int r_tile,
                                           int t_tile, float* lds) {
   using C = Chunk<KW>;
-  constexpr int RW = 4 / KW, M = PAIR ? 2 : 1;
-  constexpr int S = 4 / KW;  // sums per lane and matrix
+  constexpr int RW = waves_of(KW) / KW, M = PAIR ? 2 : 1;
+  constexpr int S = KW == 8 ? 1 : 4 / KW;  // sums per lane and matrix
   constexpr int TU = F::kUnitTerms, UW = C::U / KW;  // a wave's units of a chunk
   constexpr int XF = x_floats<F, KW>(), TF = term_floats<F, KW, M>();
   static_assert(UW * KW == C::U, "a chunk's units divide among the waves");
@@ -438,14 +440,14 @@ __device__ __forceinline__ void gemm_body(const GemvArgs& a, const BatchShape& b
     }
     if (more) stage_x(lds + ((chunk + 1) & 1) * XF);
     __syncthreads();
-    if constexpr (KW > 1) {
+    if (KW > 1 && kw * S < 4) {
       const int left = a.terms - chunk * C::U * TU;
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         const float* o = xch + (rw * C::U * TU * M + m) * 256 + 4 * lane + kw * S;
 #pragma unroll
         for (int g = 0; g < C::U * TU; ++g) {
-          if (F::kHalf && g >= left) break;
+          if ((F::kHalf || C::K > 256) && g >= left) break;
           if constexpr (S == 1) {
             sum[m][0] = sum[m][0] + o[g * M * 256];
           } else {
@@ -472,6 +474,7 @@ __device__ __forceinline__ void gemm_body(const GemvArgs& a, const BatchShape& b
 #pragma unroll 1
     for (int chunk = 0; chunk < chunks; ++chunk) body(chunk, std::integral_constant<int, 0>{});
   }
+  if (kw * S >= 4) return;
 #pragma unroll
   for (int i = 0; i < S; ++i) {
     const int tok = tk0 + 4 * s + kw * S + i;
@@ -501,7 +504,7 @@ __device__ __forceinline__ bool tile_of(int row_tiles, int tok_tiles, int& r_til
 }
 
 template <class F, int KW, bool PAIR>
-__global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemvArgs a, BatchShape b) {
+__global__ __launch_bounds__(64 * waves_of(KW)) void gemm_mfma_kernel(GemvArgs a, BatchShape b) {
   extern __shared__ __align__(16) float lds[];
   int r_tile, t_tile;
   if (tile_of(b.row_tiles, b.tok_tiles, r_tile, t_tile))
@@ -520,7 +523,7 @@ struct MultiBatch {
 };
 
 template <int KW, bool Q8>
-__global__ __launch_bounds__(kThreads) void gemm_mfma_multi_kernel(MultiBatch m) {
+__global__ __launch_bounds__(64 * waves_of(KW)) void gemm_mfma_multi_kernel(MultiBatch m) {
   extern __shared__ __align__(16) float lds[];
   int r_tile, t_tile;
   if (!tile_of(m.row_tiles, m.shape[0].tok_tiles, r_tile, t_tile)) return;
@@ -534,7 +537,19 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_multi_kernel(MultiBatch m)
     gemm_body<Q6KM, KW, false>(m.seg[i], m.shape[i], r_tile, t_tile, lds);
 }
 
+constexpr size_t kLds = 160 << 10;  // of a CU
+
 int cu_count() { return ctx().num_cus > 0 ? ctx().num_cus : 256; }
+
+// Eight waves on a row tile: where the launch's tiles leave CUs idle, two waves
+// a SIMD instead of one hide each other's MFMA and LDS waits; not for rows of
+// a chunk or two, and a Q6_K pair's exchanged terms don't fit the LDS.
+// Measured, us for 8 / 4 waves: n = 2048, 128 tiles, Q4_K 9.4 / 11.5, Q6_K 11.9 /
+// 13.7, Q8_0 12.0 / 14.5; n = 5632 20.1 / 27.9; n = 512 4.4 / 4.4 (Q6_K 5.7 / 5.4);
+// 384 tiles of n = 2048 17.6 / 15.7.
+bool eight_waves(const GemvArgs& a, long tiles, bool q6_pair) {
+  return tiles <= cu_count() && a.n >= 1024 && !q6_pair;
+}
 
 // Waves per row tile, from the launch's 16 x 16 tiles (a pair's count once):
 // the most that still adds waves to idle SIMDs.  Measured, us at n = 2048,
@@ -542,7 +557,8 @@ int cu_count() { return ctx().num_cus > 0 ? ctx().num_cus : 256; }
 // 1408 35 / 32 / 37, 5632 114 / 95 / 94; Q6_K 256 13.6 / 21 / 28, 1024 36 /
 // 32 / 30, 5632 179 / 142 / 137.  Q8_0's products keep four tiles of
 // registers each and spill the unsplit form: 5632 tiles 179 / 156 / 213.
-int waves_per_tile(long tiles, bool q8) {
+int waves_per_tile(const GemvArgs& a, long tiles, bool q8, bool q6_pair) {
+  if (eight_waves(a, tiles, q6_pair)) return 8;
   const int cus = cu_count();
   if (tiles < 4L * cus) return 4;
   return tiles < 8L * cus || q8 ? 2 : 1;
@@ -553,7 +569,8 @@ BatchShape shape_of(const GemvArgs& a, int n_tok, int x_stride, int out_stride, 
   b.n_tok = n_tok;
   b.x_stride = x_stride;
   b.out_stride = out_stride;
-  b.row_tiles = (a.d + kMT * (4 / kw) - 1) / (kMT * (4 / kw));
+  const int rows = kMT * (waves_of(kw) / kw);
+  b.row_tiles = (a.d + rows - 1) / rows;
   b.tok_tiles = (n_tok + kMT - 1) / kMT;
   return b;
 }
@@ -568,17 +585,20 @@ long tiles_of(const GemvArgs& a, int n_tok) {
 
 template <class F, int KW>
 void launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
-  const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(kThreads);
-  if (pair)
-    hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, true>), grid, block, (lds_bytes<F, KW, true>()),
-                       st, a, b);
-  else
+  const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(64 * waves_of(KW));
+  if (!pair) {
     hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, false>), grid, block, (lds_bytes<F, KW, false>()),
                        st, a, b);
+  } else if constexpr (lds_bytes<F, KW, true>() <= kLds) {
+    hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, true>), grid, block, (lds_bytes<F, KW, true>()),
+                       st, a, b);
+  }
 }
 template <class F>
 void launch_f(int kw, bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
-  if (kw == 4) {
+  if (kw == 8) {
+    launch_k<F, 8>(pair, a, b, st);
+  } else if (kw == 4) {
     launch_k<F, 4>(pair, a, b, st);
   } else if (F::kHalf || kw == 2) {  // Q8_0: waves_per_tile has no 1
     launch_k<F, 2>(pair, a, b, st);
@@ -592,7 +612,8 @@ void launch_multi(const MultiBatch& m, hipStream_t st) {
   const size_t lds = Q8 ? lds_bytes<Q80M, KW, false>()
                         : std::max(lds_bytes<Q4KM, KW, false>(), lds_bytes<Q6KM, KW, false>());
   hipLaunchKernelGGL((gemm_mfma_multi_kernel<KW, Q8>),
-                     dim3(grid_of(m.row_tiles, m.shape[0].tok_tiles)), dim3(kThreads), lds, st, m);
+                     dim3(grid_of(m.row_tiles, m.shape[0].tok_tiles)), dim3(64 * waves_of(KW)), lds,
+                     st, m);
 }
 
 }  // namespace
@@ -601,22 +622,24 @@ namespace plh {
 
 // The estimates, in us, are fits to measured times of both kernels (n 256 to
 // 11008, d 65 to 11264, 2 to 128 tokens, warm): the VALU kernel's 6 to 8 plus
-// its work per weight and token; here a wave's chain of units (0.26 a unit
-// with four waves on a row, whatever the number of rows) or, with the chip
-// full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and 2 / 4 / 17
-// / 128 tokens the two take 8.7 / 12.2 / 20 / 70 and 10.9 / 10.9 / 11.2 / 25 us,
-// at n = 11008, d = 129 and 40 tokens 18.4 and 48.6.
+// its work per weight and token; here a wave's chain of units (0.21 or 0.26 a
+// unit with eight or four waves on a row, whatever the number of rows) or, with
+// the chip full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and
+// 2 / 4 / 16 / 128 tokens the two take 8.7 / 12.2 / 19 / 70 and 9.4 / 9.4 / 9.4 /
+// 25 us.
 bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
   const double w = 1e-6 * a.n * (double)a.d * (pair ? 2 : 1);
   const bool q4 = qtype == kTypeQ4K, q8 = qtype == kTypeQ8_0;
   const double valu = (q8 ? 6.0 : 8.0) + w * n_tok * (q4 ? 0.12 : q8 ? 0.125 : 0.22);
   const double work = w * ((n_tok + kMT - 1) / kMT * kMT) * (q4 ? 0.032 : q8 ? 0.053 : 0.046);
-  const double chain = 0.26 * ((a.n + 63) / 64) * (pair ? 2 : 1);
+  const double unit = eight_waves(a, tiles_of(a, n_tok), pair && qtype == kTypeQ6K) ? 0.21 : 0.26;
+  const double chain = unit * ((a.n + 63) / 64) * (pair ? 2 : 1);
   return 2.5 + std::max(chain, work) < valu;
 }
 
 int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride) {
-  const int kw = waves_per_tile(tiles_of(a, n_tok), qtype == kTypeQ8_0);
+  const int kw = waves_per_tile(a, tiles_of(a, n_tok), qtype == kTypeQ8_0,
+                                pair && qtype == kTypeQ6K);
   const BatchShape b = shape_of(a, n_tok, x_stride, out_stride, kw);
   hipStream_t st = ctx().stream;
   if (qtype == kTypeQ4K)
@@ -639,7 +662,7 @@ int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride
   long tiles = 0;
   for (int i = 0; i < 3; ++i) tiles += tiles_of(a[i], n_tok);
   const bool q8 = qtype[0] == kTypeQ8_0;
-  const int kw = waves_per_tile(tiles, q8);
+  const int kw = waves_per_tile(a[0], tiles, q8, false);
   for (int i = 0; i < 3; ++i) {
     m.seg[i] = a[i];
     m.qtype[i] = qtype[i];
@@ -650,12 +673,16 @@ int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride
   m.row_tiles = m.tile2 + m.shape[2].row_tiles;
   hipStream_t st = ctx().stream;
   if (q8) {  // never with one wave (waves_per_tile)
-    if (kw == 2)
+    if (kw == 8)
+      launch_multi<8, true>(m, st);
+    else if (kw == 2)
       launch_multi<2, true>(m, st);
     else
       launch_multi<4, true>(m, st);
   } else if (kw == 1) {
     launch_multi<1, false>(m, st);
+  } else if (kw == 8) {
+    launch_multi<8, false>(m, st);
   } else if (kw == 2) {
     launch_multi<2, false>(m, st);
   } else {

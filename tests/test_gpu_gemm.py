@@ -1,6 +1,7 @@
 """The batched GEMV (plh_matmul_batch) on the matrix cores, bit for bit against
 the oracle's vec_dot per (row, token): every waves-per-row-tile form (chosen by
-the number of 16 x 16 tiles: below 1024 four waves, below 2048 two, else one),
+the number of 16 x 16 tiles: to 256 eight waves where rows are of 1024 or more,
+below 1024 four, below 2048 two, else one),
 rows and tokens that leave partial tiles, rows of one unit, of one chunk, of an
 odd number of blocks (Q8_0's half unit), and the shapes that stay on the VALU
 kernel.  Subnormal and huge activations, and infinities and NaNs that must stay
@@ -10,6 +11,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+from attn_check import FWD_TOL_FAST
 from picolm_amd import gemv as G
 from picolm_amd import synth as S
 
@@ -39,6 +41,8 @@ def assert_bits(got, want, what):
     (Q4, 256, 1, 16), (Q4, 256, 77, 33), (Q4, 512, 16, 15), (Q4, 768, 65, 17), (Q4, 2048, 200, 5),
     (Q6, 256, 3, 19), (Q6, 512, 33, 16), (Q6, 1280, 130, 31), (Q6, 2048, 64, 6),
     (Q8, 32, 5, 20), (Q8, 64, 16, 16), (Q8, 96, 100, 37), (Q8, 288, 17, 18), (Q8, 1056, 64, 33),
+    (Q4, 1280, 64, 17), (Q4, 1536, 40, 16), (Q6, 1024, 50, 16), (Q6, 2304, 33, 31),  # eight
+    (Q8, 1184, 48, 33), (Q8, 2080, 17, 16), (Q4, 2048, 2048, 32), (Q4, 2048, 2049, 32),
     (Q4, 256, 8200, 32), (Q6, 256, 8200, 32), (Q8, 160, 8200, 32),     # two waves a tile
     (Q4, 512, 16400, 31), (Q6, 256, 16400, 32), (Q8, 96, 16400, 32),   # one (Q8_0 two)
     (Q4, 11008, 65, 5), (Q6, 11008, 20, 3), (Q8, 11008, 33, 4)])       # the VALU kernel
@@ -118,3 +122,25 @@ def test_prompt_qkv_launches(gpu, oracle_mod, q, k, v, n_tok):
     """q, k and v of a prompt: K quants or Q8_0 in one launch, mixed in three."""
     types = dict(embd=Q8, output=Q8, q=q, k=k, v=v, o=Q4, gate=Q4, up=Q4, down=Q4)
     layer0_rows_exact(gpu, oracle_mod, n_tok, n_embd=768, types=types)
+
+
+@pytest.mark.parametrize("n_embd,gate", [(1280, Q4), (1536, Q6), (1312, Q8)])
+@pytest.mark.parametrize("n_tok", [17, 60])
+def test_prompt_long_rows_few_tiles(gpu, oracle_mod, n_embd, gate, n_tok):
+    """A layer's q/k/v launch and gate/up pair of few tiles and long rows: the
+    residual and the logits (the fast order) against the oracle."""
+    types = dict(embd=Q8, output=Q8, q=Q8, k=Q8, v=Q8, o=Q8, gate=gate, up=gate, down=Q8)
+    cfg = dict(n_layers=1, n_embd=n_embd, n_ffn=512, n_heads=4, n_kv_heads=2, head_dim=64,
+               vocab_size=64, max_seq_len=80, rope_type=0, rope_base=1e4, eps=1e-5, types=types)
+    h = S.SynthModel(**cfg, seed=n_tok)
+    dm, orc = gpu.DeviceModel(h), oracle_mod.OracleForward(h)
+    toks = np.arange(n_tok, dtype=np.int32)
+    try:
+        dm.prefill(toks, 0)
+        gpu.synchronize()
+        for got, want in zip((dm.fetch_logits(), dm.fetch_x()), orc.prefill(toks, 0, n_threads=8)):
+            assert np.max(np.abs(got - want)) <= FWD_TOL_FAST * np.max(np.abs(want))
+        for a, b in zip(dm.fetch_cache(), (orc.kc, orc.vc)):
+            assert np.array_equal(a, b)
+    finally:
+        dm.free()
