@@ -38,7 +38,7 @@
 // MFMAs.  One workgroup per token and q head on the VALU, which this replaced,
 // against this, us a layer: decode at head_dim 80, 32 heads, pos 1499: 133
 // (with its append launch) -> 9.7; 300-token prompt at head_dim 96, 32 q and 8
-// kv heads: 84 -> 18 (8 layers in one launch: 9.3 each).  The same on
+// kv heads: 84 -> 16 (8 layers in one launch: 8.4 each).  The same on
 // v_mfma_f32_16x16x4_f32 without parts: 10.8, 27 and 13.4.  Relative error
 // against 64 bits, before -> now: 2.4e-7 -> 2.0e-7 and 1.6e-7 -> 1.3e-7.
 #include <algorithm>
@@ -72,7 +72,6 @@ struct GenericArgs {
   uint16_t* v_rows;
   int layer0, n_launch_layers, n_heads, n_kv_heads, D, max_seq_len, rope_type;
   int start_pos, n_tokens, out_stride;
-  int fuse;                        // decode: append row start_pos in this launch
   int col_tiles;                   // 16-column tiles per kv head
   int n_split, split_len;          // key ranges per tile (split_len a multiple of 32)
   int n_chunk;                     // append: workgroups per (layer, token)
@@ -255,8 +254,14 @@ __device__ __forceinline__ void clear_past(int D, int g, u32x4_t (&r)[DK]) {
   }
 }
 
-template <int DT, int KS, bool D8>
-__global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) {
+// ONE: a single token, whose row is appended here (KS 4).  Prompts at head dims
+// 65 to 96 ask for registers for three workgroups a CU: 300 tokens at head_dim
+// 96, 32 q and 8 kv heads, 17.5 -> 16.4 us with the append (at 64 the compiler
+// gets there by itself, at 128 it cannot; a decode's few workgroups lose 2%).
+template <int DT, int KS, bool D8, bool ONE>
+__global__ __launch_bounds__(kGThreads, !ONE && D8 && (DT == 5 || DT == 6) ? 3 : 1) void
+generic_attn_kernel(GenericArgs a) {
+  static_assert(!ONE || KS == 4, "NewRow::finish has barriers: one column tile a workgroup");
   using Sh = GShape<DT, KS>;
   constexpr int DK = Sh::DK, CW = Sh::CW, NC = 16 * CW;
   extern __shared__ __align__(16) float lds[];
@@ -272,7 +277,7 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
   PLH_ARGS_NOW("s"(a.q), "s"(a.k), "s"(a.v), "s"(a.kc), "s"(a.vc), "s"(a.cos_t), "s"(a.sin_t),
                "s"(a.qn), "s"(a.kn), "s"(a.layer0), "s"(a.n_heads), "s"(a.n_kv_heads), "s"(a.D),
                "s"(a.max_seq_len), "s"(a.rope_type), "s"(a.start_pos), "s"(a.n_tokens),
-               "s"(a.fuse), "s"(a.col_tiles), "s"(a.n_split), "s"(a.split_len),
+               "s"(a.col_tiles), "s"(a.n_split), "s"(a.split_len),
                "s"(a.fd_split.m), "s"(a.fd_split.sh), "s"(a.fd_tiles.m));
   const int D = a.D, kv_dim = a.n_kv_heads * D;
   const int G = (int)fdiv(a.n_heads, a.fd_kvh);
@@ -295,10 +300,9 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
   const size_t layer_off = (size_t)(a.layer0 + li) * a.max_seq_len * kv_dim + (size_t)kvh * D;
   const uint16_t* kl = a.kc + layer_off;
   const uint16_t* vl = a.vc + layer_off;
-  // KS 4: every wave has the workgroup's one column tile (finish has barriers)
-  const bool own = KS == 4 && a.fuse && t0 < te && te == kmax;  // appends row start_pos
+  const bool own = ONE && t0 < te && te == kmax;  // appends row start_pos
   // rows this workgroup reads from the cache: below te, and below the new row
-  const int rmax = max((a.fuse ? min(te, a.start_pos) : te) - 1, 0);
+  const int rmax = max((ONE ? min(te, a.start_pos) : te) - 1, 0);
 
   // ---- loads: the new row's inputs, q, then the first tile --------------------
   const size_t nsrc = (size_t)li * kv_dim + (size_t)kvh * D;
@@ -394,8 +398,9 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
       }
     }
   }
-  const int lim = a.start_pos + (int)fdiv(c0 + max(min(c, nc - 1), 0), a.fd_g);  // column c's last key
-  const int lim0 = a.start_pos + (int)fdiv(c0, a.fd_g);                  // the first column's
+  // the last key of column c and of the first column
+  const int lim = a.start_pos + (int)fdiv(c0 + max(min(c, nc - 1), 0), a.fd_g);
+  const int lim0 = a.start_pos + (int)fdiv(c0, a.fd_g);
   const float up = ups[16 * cw + c];
   qs += cw * Sh::kQ;
 
@@ -454,7 +459,8 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
           const _Float16* qp = qs + c * Sh::QP + 32 * j + 8 * g;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float q = (float)qp[e] + ((float)qp[16 * Sh::QP + e] + (float)qp[32 * Sh::QP + e]);
+            const float q =
+                (float)qp[e] + ((float)qp[16 * Sh::QP + e] + (float)qp[32 * Sh::QP + e]);
             s[0] = mfma_f32((float)__builtin_bit_cast(half8_t, ka[j])[e], q, s[0]);
             s[1] = mfma_f32((float)__builtin_bit_cast(half8_t, kb[j])[e], q, s[1]);
           }
@@ -497,20 +503,25 @@ __global__ __launch_bounds__(kGThreads) void generic_attn_kernel(GenericArgs a) 
         const half8_t bh = cat(ph), bm = cat(pm), bl = cat(pl);
         // keys 4 g + v and 16 + 4 g + v of 16 d's: the order of P's registers
         const _Float16* vr = vt + (4 * g + (c >> 2)) * Sh::VP + 4 * (c & 3);
-        half8_t vv[DT];
+        constexpr int H = 3;  // d tiles whose V operands are in registers together
 #pragma unroll
-        for (int j = 0; j < DT; ++j) {
-          const half4_t v0 = lds_read_tr4(vr + 16 * j);
-          const half4_t v1 = lds_read_tr4(vr + 16 * Sh::VP + 16 * j);
-          vv[j] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
+        for (int j0 = 0; j0 < DT; j0 += H) {
+          half8_t vv[H];
 #pragma unroll
-        for (int j = 0; j < DT; ++j) {
-          float4_t x = {0.f, 0.f, 0.f, 0.f};
-          x = mfma16x16x32(vv[j], bl, x);
-          x = mfma16x16x32(vv[j], bm, x);
-          x = mfma16x16x32(vv[j], bh, x);
-          o[j] = o[j] + x;
+          for (int j = j0; j < j0 + H && j < DT; ++j) {
+            const half4_t v0 = lds_read_tr4(vr + 16 * j);
+            const half4_t v1 = lds_read_tr4(vr + 16 * Sh::VP + 16 * j);
+            vv[j - j0] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
+#pragma unroll
+          for (int j = j0; j < j0 + H && j < DT; ++j) {
+            float4_t x = {0.f, 0.f, 0.f, 0.f};
+            x = mfma16x16x32(vv[j - j0], bl, x);
+            x = mfma16x16x32(vv[j - j0], bm, x);
+            x = mfma16x16x32(vv[j - j0], bh, x);
+            o[j] = o[j] + x;
+          }
+          asm volatile("" ::: "memory");
         }
       } else {
 #pragma unroll 1
@@ -657,37 +668,38 @@ int built_tiles(int head_dim) {
   return t <= 6 ? t : t <= 8 ? 8 : t <= 10 ? 10 : t <= 12 ? 12 : 16;
 }
 
-template <int DT, int KS>
+template <int DT, int KS, bool ONE>
 void launch_attn_ks(const GenericArgs& a, unsigned grid, hipStream_t st) {
   constexpr size_t lds = sizeof(float) * GShape<DT, KS>::kFloats;
   // 16-byte loads where every row starts on 16 bytes
   if (a.D % 8 == 0 && ((uintptr_t)a.kc | (uintptr_t)a.vc) % 16 == 0)
-    hipLaunchKernelGGL((generic_attn_kernel<DT, KS, true>), dim3(grid), dim3(kGThreads), lds, st,
-                       a);
+    hipLaunchKernelGGL((generic_attn_kernel<DT, KS, true, ONE>), dim3(grid), dim3(kGThreads), lds,
+                       st, a);
   else
-    hipLaunchKernelGGL((generic_attn_kernel<DT, KS, false>), dim3(grid), dim3(kGThreads), lds, st,
-                       a);
+    hipLaunchKernelGGL((generic_attn_kernel<DT, KS, false, ONE>), dim3(grid), dim3(kGThreads), lds,
+                       st, a);
 }
 template <int DT>
-void launch_attn(const GenericArgs& a, int ks, unsigned grid, hipStream_t st) {
+void launch_attn(const GenericArgs& a, bool one, int ks, unsigned grid, hipStream_t st) {
+  if (one) return launch_attn_ks<DT, 4, true>(a, grid, st);
   if constexpr (two_tiles(DT)) {
-    if (ks == 2) return launch_attn_ks<DT, 2>(a, grid, st);
+    if (ks == 2) return launch_attn_ks<DT, 2, false>(a, grid, st);
   }
-  launch_attn_ks<DT, 4>(a, grid, st);
+  launch_attn_ks<DT, 4, false>(a, grid, st);
 }
 
-void launch_attn(const GenericArgs& a, int ks, unsigned grid, hipStream_t st) {
+void launch_attn(const GenericArgs& a, bool one, int ks, unsigned grid, hipStream_t st) {
   switch (built_tiles(a.D)) {
-    case 1: launch_attn<1>(a, ks, grid, st); break;
-    case 2: launch_attn<2>(a, ks, grid, st); break;
-    case 3: launch_attn<3>(a, ks, grid, st); break;
-    case 4: launch_attn<4>(a, ks, grid, st); break;
-    case 5: launch_attn<5>(a, ks, grid, st); break;
-    case 6: launch_attn<6>(a, ks, grid, st); break;
-    case 8: launch_attn<8>(a, ks, grid, st); break;
-    case 10: launch_attn<10>(a, ks, grid, st); break;
-    case 12: launch_attn<12>(a, ks, grid, st); break;
-    default: launch_attn<16>(a, ks, grid, st); break;
+    case 1: launch_attn<1>(a, one, ks, grid, st); break;
+    case 2: launch_attn<2>(a, one, ks, grid, st); break;
+    case 3: launch_attn<3>(a, one, ks, grid, st); break;
+    case 4: launch_attn<4>(a, one, ks, grid, st); break;
+    case 5: launch_attn<5>(a, one, ks, grid, st); break;
+    case 6: launch_attn<6>(a, one, ks, grid, st); break;
+    case 8: launch_attn<8>(a, one, ks, grid, st); break;
+    case 10: launch_attn<10>(a, one, ks, grid, st); break;
+    case 12: launch_attn<12>(a, one, ks, grid, st); break;
+    default: launch_attn<16>(a, one, ks, grid, st); break;
   }
 }
 
@@ -718,7 +730,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // 512 workgroups: 15.5 / 11.3 / 13.5 / 12.6), as far as every wave keeps a
   // tile, the partials fit the static scratch and the merges its counters.
   const int G = n_heads / n_kv_heads, cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  a.fuse = append && n_tokens == 1;
+  const bool one = append && n_tokens == 1;
   const int dt = built_tiles(head_dim), kmax = start_pos + n_tokens;
   const long tiles = (long)n_kv_heads * ((n_tokens * G + 15) / 16) * n_launch_layers;
   // Two column tiles a workgroup halve its fixed chain per column but give a
@@ -726,7 +738,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // 96, 32 q and 8 kv heads, 8 layers, KS 2 / 4: 128 tokens 28.3 / 34.8 us, 300
   // 70.3 / 83.0, 500 149 / 159; one layer of 1500 tokens 138 / 125, of 300 21.6 /
   // 18.7).  Up to head_dim 64 both take the same.
-  const int ks = !a.fuse && two_tiles(dt) && tiles >= 4L * cus && kmax <= 512 ? 2 : 4;
+  const int ks = !one && two_tiles(dt) && tiles >= 4L * cus && kmax <= 512 ? 2 : 4;
   a.col_tiles = (n_tokens * G + 64 / ks - 1) / (64 / ks);
   const long groups_layer = (long)n_kv_heads * a.col_tiles;
   unsigned* ctr = nullptr;
@@ -780,7 +792,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
     if (k_rows) b.k_rows = k_rows + rows_before * kv_dim;
     if (v_rows) b.v_rows = v_rows + rows_before * kv_dim;
     const long nl = b.n_launch_layers;
-    if (append && !a.fuse) {
+    if (append && !one) {
       const long rows = nl * n_tokens * n_kv_heads;
       if (b.kn)
         hipLaunchKernelGGL(generic_append_norm_kernel, dim3((unsigned)rows), dim3(kGThreads), 0,
@@ -790,7 +802,7 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
                            dim3(kGThreads), 0, st, b);
       if (check_hip(hipGetLastError(), "generic_append_kernel")) return -1;
     }
-    launch_attn(b, ks, (unsigned)(nl * groups_layer * a.n_split), st);
+    launch_attn(b, one, ks, (unsigned)(nl * groups_layer * a.n_split), st);
     if (check_hip(hipGetLastError(), "generic_attn_kernel")) return -1;
   }
   return 0;
