@@ -38,7 +38,7 @@
 // MFMAs.  One workgroup per token and q head on the VALU, which this replaced,
 // against this, us a layer: decode at head_dim 80, 32 heads, pos 1499: 133
 // (with its append launch) -> 9.7; 300-token prompt at head_dim 96, 32 q and 8
-// kv heads: 84 -> 16 (8 layers in one launch: 8.4 each).  The same on
+// kv heads: 84 -> 16 (8 layers in one launch: 8.1 each).  The same on
 // v_mfma_f32_16x16x4_f32 without parts: 10.8, 27 and 13.4.  Relative error
 // against 64 bits, before -> now: 2.4e-7 -> 2.0e-7 and 1.6e-7 -> 1.3e-7.
 #include <algorithm>
@@ -734,10 +734,11 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   const int dt = built_tiles(head_dim), kmax = start_pos + n_tokens;
   const long tiles = (long)n_kv_heads * ((n_tokens * G + 15) / 16) * n_launch_layers;
   // Two column tiles a workgroup halve its fixed chain per column but give a
-  // wave twice the tiles: faster with many workgroups and few keys (head_dim
-  // 96, 32 q and 8 kv heads, 8 layers, KS 2 / 4: 128 tokens 28.3 / 34.8 us, 300
-  // 70.3 / 83.0, 500 149 / 159; one layer of 1500 tokens 138 / 125, of 300 21.6 /
-  // 18.7).  Up to head_dim 64 both take the same.
+  // wave twice the tiles: faster with many workgroups and few keys (32 q and 8
+  // kv heads, 8 layers in a launch, KS 2 / 4, us: head_dim 96, 128 tokens 26.2 /
+  // 28.2, 300 64.8 / 69.2, 500 130 / 138, head_dim 112, 300 tokens 85.7 / 100.4; one
+  // layer of 300 tokens 16.8 / 15.6, of 1500 116 / 115).  Up to head_dim 64 both
+  // take the same.
   const int ks = !one && two_tiles(dt) && tiles >= 4L * cus && kmax <= 512 ? 2 : 4;
   a.col_tiles = (n_tokens * G + 64 / ks - 1) / (64 / ks);
   const long groups_layer = (long)n_kv_heads * a.col_tiles;
