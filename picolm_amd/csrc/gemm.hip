@@ -18,10 +18,10 @@
 // What bounds it: the fp32 MFMA and the VALU share one pipe (measured: a
 // 16x16x4 takes 32 cycles, and VALU instructions between them add their 4
 // cycles each), so a 16 x 16 tile of a 64-element Q4_K unit costs 16 x 32
-// MFMA cycles + ~150 x 4 VALU cycles (88 of them the exact order's own adds
+// MFMA cycles + ~120 x 4 VALU cycles (88 of them the exact order's own adds
 // and products).  TinyLlama's 128-token prompt, us a launch before (the VALU
-// kernel) and now: gate/up pair (5632 x 2048 Q4_K twice) 340 -> 96, down (2048 x
-// 5632 Q6_K) 287 -> 77, o 70 -> 25, q, k and v 102 in three launches -> 36 in
+// kernel) and now: gate/up pair (5632 x 2048 Q4_K twice) 340 -> 93, down (2048 x
+// 5632 Q6_K) 287 -> 76, o 70 -> 26, q, k and v 102 in three launches -> 34 in
 // one; the whole prompt 18.1 -> 5.5 ms.  Set aside: x straight from the caches
 // instead of LDS (Q4_K 11264 x 2048, 128 tokens: 136 us against 96, Q6_K 387
 // against 130: the vector memory path handles the 16 tokens' lines one by
