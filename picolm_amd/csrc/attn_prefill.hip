@@ -797,13 +797,18 @@ int g_prefill_ksplit = 0;
 // 21.1), and so do long contexts, by wave tiles (32 keys, 16 columns) per CU:
 // above about 50 at head_dim 64 (128 tokens at start 8000: 55 -> 67 us) and 20
 // at 128 (200 tokens at start 1000: 29 -> 33), unless the unit's columns fill
-// one wave in four at most (2 tokens at start 8000, 22 layers: 125 -> 49).
+// one wave in four at most (2 tokens at start 8000, 22 layers: 125 -> 49; at
+// head_dim 128 two tiles then read each K/V row twice: 28 columns, 112 units 58 ->
+// 42, but 20 columns, 512 units 73 -> 80).
 // Prompts within two key tiles take either way the same time.
 static bool few_tiles_pay(const PrefillArgs& a, int head_dim, int cus) {
   if (g_prefill_split || g_prefill_ksplit) return false;  // the units' own splits, by tuning
   const long G = a.n_heads / a.n_kv_heads, cols = a.n_tokens * G;
   const long key_tiles = (a.start_pos + a.n_tokens + kKT - 1) / kKT;
-  if (a.n_tokens == 1 || (cols <= 32 && key_tiles > 8)) return true;
+  if (a.n_tokens == 1) return true;
+  if (key_tiles > 8 &&
+      (cols <= 16 || (cols <= 32 && (head_dim == 64 || (long)a.n_units * 2 <= cus))))
+    return true;
   const double tiles = (double)a.n_launch_layers * a.n_kv_heads * ((cols + 15) / 16) *
                        (a.start_pos + 0.5 * a.n_tokens) / kKT;
   return (long)a.n_units * 4 <= cus && key_tiles >= 3 &&

@@ -77,7 +77,9 @@ FEW = [  # n_layers, n_heads, n_kv_heads, head_dim, rope_type, qk_norm, start, n
     (1, 14, 2, 64, 0, True, 300, 1, 0), (1, 32, 4, 64, 1, False, 0, 65, 4),
     (1, 14, 2, 64, 1, True, 200, 100, 0), (1, 16, 8, 128, 1, True, 0, 509, 0),
     (1, 28, 4, 128, 0, False, 17, 80, 8), (22, 12, 4, 64, 0, False, 260, 10, 0),
-    (9, 16, 8, 128, 1, True, 400, 16, 0), (1, 128, 1, 64, 0, False, 90, 6, 0)]
+    (9, 16, 8, 128, 1, True, 400, 16, 0),
+    (16, 8, 8, 128, 0, False, 300, 16, 0), (3, 16, 8, 128, 1, True, 300, 10, 4),
+    (1, 128, 1, 64, 0, False, 90, 6, 0)]
 
 
 @pytest.mark.parametrize("case", FEW)
