@@ -336,8 +336,9 @@ constexpr size_t lds_bytes() {
 // for a gate/up pair).  The waves take row tiles of their own (KW 1), or KW
 // waves share a row tile: each forms the terms of a KW-th of a chunk's units
 // into LDS, then chains a KW-th of the tile's sums (KW 8: the first four waves a
-// quarter) over the chunk's terms, in block order.  One barrier per chunk; the next chunk's x, the next unit's operand
-// and the weights of the next two units are in flight meanwhile.
+// quarter) over the chunk's terms, in block order.  One barrier per chunk; the
+// next chunk's x, the next unit's operand and the weights of the next two units
+// are in flight meanwhile.
 template <class F, int KW, bool PAIR>
 __device__ __forceinline__ void gemm_body(const GemvArgs& a, const BatchShape& b, int r_tile,
                                           int t_tile, float* lds) {
@@ -621,20 +622,26 @@ void launch_multi(const MultiBatch& m, hipStream_t st) {
 namespace plh {
 
 // The estimates, in us, are fits to measured times of both kernels (n 256 to
-// 11008, d 65 to 11264, 2 to 128 tokens, warm): the VALU kernel's 6 to 8 plus
-// its work per weight and token; here a wave's chain of units (0.21 or 0.26 a
-// unit with eight or four waves on a row, whatever the number of rows) or, with
-// the chip full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and
-// 2 / 4 / 16 / 128 tokens the two take 8.7 / 12.2 / 19 / 70 and 9.4 / 9.4 / 9.4 /
-// 25 us.
+// 11008, d 65 to 11264, 2 to 128 tokens, warm): the VALU kernel's latency (a group
+// of four tokens takes longer than two) or its work per weight and token; here
+// a wave's chain of units, longer with every further tile a CU (its workgroups
+// share the SIMDs; from four a CU on fewer waves share a tile), or, with the chip
+// full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and 2 / 4 / 16 /
+// 128 tokens the two take 8.7 / 12.2 / 19 / 70 and 9.4 / 9.4 / 9.4 / 25 us; at 2304
+// x 6743 Q6_K and 2 tokens (two tiles a CU) 13.8 and 20.4.
 bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
   const double w = 1e-6 * a.n * (double)a.d * (pair ? 2 : 1);
   const bool q4 = qtype == kTypeQ4K, q8 = qtype == kTypeQ8_0;
-  const double valu = (q8 ? 6.0 : 8.0) + w * n_tok * (q4 ? 0.12 : q8 ? 0.125 : 0.22);
+  const double least = q4 ? (n_tok > 3 ? 11.5 : 8) : q8 ? (n_tok > 3 ? 8 : 6) : n_tok > 2 ? 12 : 10;
+  const double valu =
+      std::max(least, (q8 ? 6.0 : 8.0) + w * n_tok * (q4 ? 0.12 : q8 ? 0.125 : 0.22));
   const double work = w * ((n_tok + kMT - 1) / kMT * kMT) * (q4 ? 0.032 : q8 ? 0.053 : 0.046);
-  const double unit = eight_waves(a, tiles_of(a, n_tok), pair && qtype == kTypeQ6K) ? 0.21 : 0.26;
+  const long tiles = tiles_of(a, n_tok), cus = cu_count();
+  const double more = (double)std::min((tiles - 1) / cus, 3L);  // tiles a CU past the first
+  double unit = q4 ? 0.28 + 0.17 * more : q8 ? 0.375 + 0.23 * more : 0.35 + 0.27 * more;
+  if (eight_waves(a, tiles, pair && qtype == kTypeQ6K)) unit = q4 ? 0.21 : 0.29;
   const double chain = unit * ((a.n + 63) / 64) * (pair ? 2 : 1);
-  return 2.5 + std::max(chain, work) < valu;
+  return 2.8 + std::max(chain, work) < valu;
 }
 
 int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride) {
