@@ -120,6 +120,9 @@ __device__ __forceinline__ void split_pair_rtz(float x0, float x1, half2_t& hi, 
 __device__ __forceinline__ float vmax(float a, float b) {
   return __builtin_elementwise_maximum(a, b);
 }
+__device__ __forceinline__ float vmin(float a, float b) {
+  return __builtin_elementwise_minimum(a, b);
+}
 
 // gfx950 transposing LDS read (ds_read_b64_tr_b16).  Within each 16-lane group,
 // lane i passes the address of 4 consecutive fp16 values: chunk i%4 of row

@@ -15,7 +15,8 @@
 //     column tile's keys and merge in LDS.  Both products run on
 //     v_mfma_f32_16x16x32_f16 with fp32 sums: K and V are fp16 already, and q
 //     (scaled by a power of two per column) and the weights go in as three
-//     fp16 parts that keep all their 24 bits.  S = K q^T with the K rows
+//     fp16 parts, the lower ones scaled up (split3): all 24 bits of weights and
+//     q elements down to 2^-36 of the column's largest.  S = K q^T with the K rows
 //     straight from the cache, O^T += V^T P^T with V^T through a wave's own
 //     LDS tile and ds_read_b64_tr_b16.  The S accumulators hold keys 4 g + v
 //     and 16 + 4 g + v of column c in lane (g, c), which is the PV operand if
@@ -42,6 +43,7 @@
 // v_mfma_f32_16x16x4_f32 without parts: 10.8, 27 and 13.4.  Relative error
 // against 64 bits, before -> now: 2.4e-7 -> 2.0e-7 and 1.6e-7 -> 1.3e-7.
 #include <algorithm>
+#include <type_traits>
 
 #include "picolm_hip.h"
 #include "attn_common.h"
@@ -192,14 +194,24 @@ __device__ __forceinline__ float4_t mfma_f32(float x, float y, float4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
 }
 
-// A pair of fp32 values (below 65504) as three fp16 parts each, x = hi + mid +
-// lo to 33 bits: hi and mid rounded toward zero, so both remainders are exact.
+// A pair of fp32 values of at most 2^14 as three fp16 parts each, every remainder
+// exact: x = hi + 2^-11 (mid + lo) keeps all 24 bits of values from 2^-11 up and
+// stops at 2^-35; DEEP, x = hi + 2^-11 (mid + 2^-11 lo), from 2^-22 up and 2^-46.
+// (Unscaled parts: from 1 up and 2^-24.)
+constexpr float kPartUp = 2048.0f, kPartDown = 1.0f / kPartUp;
+template <bool DEEP>
 __device__ __forceinline__ void split3(float x0, float x1, half2_t& hi, half2_t& mid,
                                        half2_t& lo) {
   const auto h = __builtin_amdgcn_cvt_pkrtz(x0, x1);
   hi = __builtin_bit_cast(half2_t, h);
-  const float r0 = x0 - (float)hi[0], r1 = x1 - (float)hi[1];
+  const float r0 = __builtin_fmaf((float)hi[0], -kPartUp, x0 * kPartUp);
+  const float r1 = __builtin_fmaf((float)hi[1], -kPartUp, x1 * kPartUp);
   split_pair_rtz(r0, r1, mid, lo);
+  if constexpr (DEEP) {
+    const float l0 = __builtin_fmaf((float)mid[0], -kPartUp, r0 * kPartUp);
+    const float l1 = __builtin_fmaf((float)mid[1], -kPartUp, r1 * kPartUp);
+    lo = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(l0, l1));
+  }
 }
 
 // Shapes for DT 16-wide tiles of d (D rounded up).  LDS: q's parts and the
@@ -366,8 +378,8 @@ generic_attn_kernel(GenericArgs a) {
     }
 #pragma unroll
     for (int m = 1; m < 16; m *= 2) amax = vmax(amax, __shfl_xor(amax, m));
-    // the column by a power of two to [2^13, 2^14), so that its three parts
-    // keep all 24 bits of every element that matters; 2^up goes to the scores
+    // the column by a power of two to [2^13, 2^14): its three parts keep all 24
+    // bits of elements down to 2^-36 of the largest; 2^up goes to the scores
     const int ex = max((int)((__float_as_uint(amax) >> 23) & 0xFFu) - 127, -100);
     const float down = __uint_as_float((uint32_t)(127 + 13 - ex) << 23);
     if (qj == 0) ups[16 * w + (tid >> 4)] = __uint_as_float((uint32_t)(127 + ex - 13) << 23);
@@ -377,7 +389,7 @@ generic_attn_kernel(GenericArgs a) {
       int i0, i1;
       pair_of(a.rope_type, D, min(qj + 16 * k, D / 2 - 1), i0, i1);
       half2_t hi, mid, lo;
-      split3(x0[w][k] * down, x1[w][k] * down, hi, mid, lo);
+      split3<true>(x0[w][k] * down, x1[w][k] * down, hi, mid, lo);
       qrow[i0] = hi[0], qrow[i1] = hi[1];
       qrow[16 * Sh::QP + i0] = mid[0], qrow[16 * Sh::QP + i1] = mid[1];
       qrow[32 * Sh::QP + i0] = lo[0], qrow[32 * Sh::QP + i1] = lo[1];
@@ -405,13 +417,18 @@ generic_attn_kernel(GenericArgs a) {
   qs += cw * Sh::kQ;
 
   // ---- the tiles ---------------------------------------------------------------
-  // Fast: fp16 MFMAs over the three parts of q and of P.  An infinity or a NaN
-  // among the rows makes a result of the wave infinite or NaN there (inf times
-  // a zero part); the wave then takes its tiles again as fp32 products that
-  // skip masked keys, which is what the rows' own values give.
+  // Fast: fp16 MFMAs over the three parts of q and of P.  The wave takes its
+  // tiles again as fp32 products that skip masked keys, which is what the rows'
+  // own values give, where
+  // - an infinity or a NaN among the rows made a result infinite or NaN (inf
+  //   times a zero part), or
+  // - some weight was below 2^-36 of the largest (the parts stop at 2^-60 of it)
+  //   and a column's result is so small that its bits could count: all of it
+  //   below 2^-16 of the largest weight, the heavier keys' V zero or nearly.
   _Float16* vt = (_Float16*)lds + CW * Sh::kQ + wave * 32 * Sh::VP;
   float4_t o[DT];
   float m, l;
+  bool lost = false;
   for (int slow = 0; slow < 2; ++slow) {
 #pragma unroll
     for (int j = 0; j < DT; ++j) o[j] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -445,7 +462,8 @@ generic_attn_kernel(GenericArgs a) {
       float4_t s[2] = {};
       if (!slow) {
 #pragma unroll
-        for (int part = 2; part >= 0; --part)
+        for (int part = 2; part >= 0; --part) {
+          if (part < 2) s[0] = s[0] * kPartDown, s[1] = s[1] * kPartDown;
 #pragma unroll
           for (int j = 0; j < DK; ++j) {
             const half8_t qf =
@@ -453,6 +471,7 @@ generic_attn_kernel(GenericArgs a) {
             s[0] = mfma16x16x32(__builtin_bit_cast(half8_t, ka[j]), qf, s[0]);
             s[1] = mfma16x16x32(__builtin_bit_cast(half8_t, kb[j]), qf, s[1]);
           }
+        }
       } else {
 #pragma unroll
         for (int j = 0; j < DK; ++j) {
@@ -460,7 +479,8 @@ generic_attn_kernel(GenericArgs a) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const float q =
-                (float)qp[e] + ((float)qp[16 * Sh::QP + e] + (float)qp[32 * Sh::QP + e]);
+                (float)qp[e] + ((float)qp[16 * Sh::QP + e] +
+                                (float)qp[32 * Sh::QP + e] * kPartDown) * kPartDown;
             s[0] = mfma_f32((float)__builtin_bit_cast(half8_t, ka[j])[e], q, s[0]);
             s[1] = mfma_f32((float)__builtin_bit_cast(half8_t, kb[j])[e], q, s[1]);
           }
@@ -468,11 +488,12 @@ generic_attn_kernel(GenericArgs a) {
       }
       load_rows(kl, t + 32 * KS, ka, kb);
       float p[8];
-      float mx = kNegBig;
+      float mx = kNegBig, least = -kNegBig;  // least: masked keys' too
       const bool cross = t + 31 > lim0;  // uniform: some key is past some column's last
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         p[i] = s[i / 4][i % 4] * up;
+        least = vmin(least, p[i]);
         if (cross && t + 16 * (i / 4) + 4 * g + i % 4 > lim) p[i] = kNegBig;
       }
       mx = vmax(vmax(vmax(p[0], p[1]), vmax(p[2], p[3])), vmax(vmax(p[4], p[5]), vmax(p[6], p[7])));
@@ -484,8 +505,9 @@ generic_attn_kernel(GenericArgs a) {
         for (int j = 0; j < DT; ++j) o[j] = o[j] * corr;
         m = mn;
       }
-      // weights times 2^14 (the sums too): every part of one stays well above
-      // fp16's smallest step
+      // weights times 2^14 (the sums too): their parts keep all 24 bits of
+      // weights down to 2^-25, the deeper ones (more VALU work) down to 2^-36
+      const bool deep = __any(least < m - 25.0f);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         p[i] = fast_exp2(p[i] - m) * 16384.0f;
@@ -493,10 +515,11 @@ generic_attn_kernel(GenericArgs a) {
       }
       l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       __builtin_amdgcn_wave_barrier();
-      if (!slow) {
+      auto pv = [&](auto deeper) {  // O^T += V^T P^T
+        constexpr bool DEEP = decltype(deeper)::value;
         half2_t ph[4], pm[4], pl[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) split3(p[2 * i], p[2 * i + 1], ph[i], pm[i], pl[i]);
+        for (int i = 0; i < 4; ++i) split3<DEEP>(p[2 * i], p[2 * i + 1], ph[i], pm[i], pl[i]);
         auto cat = [](const half2_t (&x)[4]) {
           return half8_t{x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
         };
@@ -517,12 +540,19 @@ generic_attn_kernel(GenericArgs a) {
           for (int j = j0; j < j0 + H && j < DT; ++j) {
             float4_t x = {0.f, 0.f, 0.f, 0.f};
             x = mfma16x16x32(vv[j - j0], bl, x);
+            if constexpr (DEEP) x = x * kPartDown;
             x = mfma16x16x32(vv[j - j0], bm, x);
-            x = mfma16x16x32(vv[j - j0], bh, x);
+            x = mfma16x16x32(vv[j - j0], bh, x * kPartDown);
             o[j] = o[j] + x;
           }
           asm volatile("" ::: "memory");
         }
+      };
+      if (!slow && !deep) {
+        pv(std::false_type{});
+      } else if (!slow) {
+        lost |= __any(least < m - 36.0f);
+        pv(std::true_type{});
       } else {
 #pragma unroll 1
         for (int key = 0; key < 32; ++key) {
@@ -543,14 +573,19 @@ generic_attn_kernel(GenericArgs a) {
       }
       __builtin_amdgcn_wave_barrier();
     }
+    if (slow) break;
     // infinite or NaN if any result is (d past D: not looked at)
-    float4_t sum = {l, 0.f, 0.f, 0.f};
+    float4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < DT; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
         if (16 * j + 16 <= D || 16 * j + 4 * g + v < D) sum[v] += fabsf(o[j][v]);
-    if (!__any(!((sum[0] + sum[1]) + (sum[2] + sum[3]) <= 3.4028235e38f))) break;
+    const float os = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    if (__any(!(l + os <= 3.4028235e38f))) continue;
+    if (!lost) break;
+    const float lc = add_xor32(add_xor16(l)), oc = add_xor32(add_xor16(os));
+    if (!__any(c < nc && lc > 0.0f && oc < 0.25f)) break;  // 2^-16 times 2^14
   }
   l = add_xor32(add_xor16(l));
 

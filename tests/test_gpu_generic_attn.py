@@ -181,6 +181,74 @@ def test_decode_infinite_cached_rows(gpu, oracle_mod, kind):
     cache.free()
 
 
+def attend64(q, k, v, group):
+    """Causal attention of the last len(q) rows in 64 bits: q [n, Hq, D], k and
+    v [rows, Hkv, D] (no rotation)."""
+    n, hq, d = q.shape
+    out = np.zeros((n, hq, d))
+    for t in range(n):
+        rows = len(k) - n + t + 1
+        for h in range(hq):
+            s = k[:rows, h // group].astype(np.float64) @ q[t, h].astype(np.float64) / np.sqrt(d)
+            w = np.exp(s - s.max())
+            out[t, h] = (w / w.sum()) @ v[:rows, h // group].astype(np.float64)
+    return out
+
+
+@pytest.mark.parametrize("D,n", [(80, 1), (48, 1), (50, 1), (96, 5), (34, 17), (64, 1), (128, 40)])
+@pytest.mark.parametrize("kind", ["w30", "w45", "w30_alone", "w80_alone", "v_zero", "q_wide"])
+def test_wide_ranges(gpu, D, n, kind):
+    """q and the softmax weights count at fp32's precision over fp32's range.
+    wB: one key's weight is 2^-B of the others' and its v 6e4 among values of
+    1e-4 (w30), the smallest fp16 (w45) or zero (alone: it is the whole
+    output); q_wide: a q element 2^30 times the others meets a channel of K
+    that is zero.  Against 64 bits, each head's 2-norm: a score of B ln 2 goes
+    through three roundings (its sum, its scale, the maximum's subtraction),
+    and a result through one per row."""
+    P = gpu
+    Hq, Hkv, start, at = 4, 2, 200, 57
+    cfg = P.AttnConfig(1, Hq, Hkv, D, start + n, 1e4, 0)
+    rng = np.random.default_rng(D + n)
+    rows = start + n
+    q = np.zeros((n, Hq, D), np.float32)
+    k, v = (np.zeros((rows, Hkv, D), np.float32) for _ in "kv")
+    bits = 4
+    if kind == "q_wide":
+        q, k, v = (normal_f32(rng, x.shape).astype(np.float16).astype(np.float32)
+                   for x in (q, k, v))
+        q[..., 3], k[..., 3] = 2.0 ** 30, 0.0
+    elif kind != "v_zero":
+        bits = int(kind[1:3])
+        q[..., 0] = np.sqrt(np.float32(D))
+        k[at, :, 0] = -bits * np.log(2.0)
+        k = k.astype(np.float16).astype(np.float32)
+        v[:] = {"w30": 1e-4, "w45": 2.0 ** -24}.get(kind, 0.0)
+        v[at] = 6e4 * rng.choice([-1.0, 1.0], (Hkv, D))
+        v = v.astype(np.float16).astype(np.float32)
+    cos, sin = (np.full((rows, D // 2), x, np.float32) for x in (1.0, 0.0))
+    cache = P.KVCache(cfg)
+    full = [np.zeros((rows, Hkv, D), np.uint16) for _ in "kv"]
+    for f, x in zip(full, (k, v)):
+        f[:start] = x[:start].astype(np.float16).view(np.uint16)
+    cache.load(*(f.reshape(-1) for f in full))
+    cache.cos.upload(cos)
+    cache.sin.upload(sin)
+    d = [P.DeviceBuffer.from_numpy(np.ascontiguousarray(x)) for x in (q, k[start:], v[start:])]
+    out = P.DeviceBuffer(4 * n * Hq * D)
+    P.prefill(cache, 0, start, n, d[0].ptr, d[1].ptr, d[2].ptr, out.ptr)
+    P.synchronize()
+    got = out.download(np.float32, (n, Hq, D)).astype(np.float64)
+    want = attend64(q, k, v, Hq // Hkv)
+    cache.free()
+    if kind == "v_zero":
+        assert not got.any()
+        return
+    err = np.linalg.norm(got - want, axis=-1) / np.linalg.norm(want, axis=-1)
+    tol = (3 * bits * np.log(2.0) + rows) * 2.0 ** -24
+    print(f"[wide] {kind} D {D} n {n}: {err.max():.2e} of {tol:.2e}", flush=True)
+    assert err.max() <= tol, (kind, err.max(), tol)
+
+
 def test_decode_capture_and_noalloc(gpu, oracle_mod):
     """A split launch captured at its first call and replayed, and the
     allocation-free entry point: the eager call's bits each time."""
