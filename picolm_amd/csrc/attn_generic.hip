@@ -751,6 +751,13 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
     return -1;
   }
   if (n_tokens == 0) return 0;
+  // A launch holds at most 2^32 - 1 threads.  First: the counts below are ints.
+  const long max_wg = 0xFFFFFFFFL / kGThreads;
+  if ((long)n_tokens * n_heads > max_wg) {
+    set_error("attention: %d tokens x %d heads exceed one launch's %ld workgroups", n_tokens,
+              n_heads, max_wg);
+    return -1;
+  }
   GenericArgs a{};
   a.q = q, a.k = k, a.v = v, a.kc = key_cache, a.vc = val_cache;
   a.cos_t = rope_cos, a.sin_t = rope_sin, a.out = out;
@@ -801,16 +808,10 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   a.fd_tiles = make_fastdiv((uint32_t)a.col_tiles);
   a.fd_kvh = make_fastdiv((uint32_t)n_kv_heads);
   a.fd_g = make_fastdiv((uint32_t)G);
-  // A launch holds at most 2^32 - 1 threads: layers go in as many launches
-  // as that takes (each layer is independent); one layer must fit.
+  // Layers go in as many launches as that takes (each is independent); one
+  // fits: n_split is 1 unless the launch has fewer groups than CUs.
   const long per_layer =
       std::max<long>(groups_layer * a.n_split, (long)n_tokens * n_kv_heads);
-  const long max_wg = 0xFFFFFFFFL / kGThreads;
-  if ((long)n_tokens * n_heads > max_wg || per_layer > max_wg) {
-    set_error("attention: %d tokens x %d heads exceed one launch's %ld workgroups", n_tokens,
-              n_heads, max_wg);
-    return -1;
-  }
   const int step = (int)std::min<long>(n_launch_layers, max_wg / per_layer);
   const size_t q_dim = (size_t)n_heads * head_dim, kv_dim = (size_t)n_kv_heads * head_dim;
   hipStream_t st = ctx().stream;

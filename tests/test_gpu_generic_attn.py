@@ -249,6 +249,18 @@ def test_wide_ranges(gpu, D, n, kind):
     assert err.max() <= tol, (kind, err.max(), tol)
 
 
+@pytest.mark.parametrize("heads,n", [(256, 1 << 24), (512, 1 << 23), (300, 1 << 23)])
+def test_sizes_past_one_launch_are_refused(gpu, heads, n):
+    """More (token, q head) pairs than a launch has workgroups, their product 0
+    modulo 2^32 or past 2^31: -1 with a message, nothing read."""
+    P = gpu
+    p = P.DeviceBuffer(256).ptr
+    rc = P.lib.plh_attn_prefill(1, heads, 1, 80, n, 0, 0, 1, 0, n, p, p, p, p, p, p, p, p,
+                                heads * 80)
+    assert rc == -1 and b"exceed one launch" in P.lib.plh_last_error()
+    P.synchronize()
+
+
 def test_decode_capture_and_noalloc(gpu, oracle_mod):
     """A split launch captured at its first call and replayed, and the
     allocation-free entry point: the eager call's bits each time."""
