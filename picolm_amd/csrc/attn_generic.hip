@@ -770,7 +770,12 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // Keys split over several workgroups where the launch would fill less than
   // one per CU (head_dim 80, 32 heads, pos 1499, us a layer for 128 / 256 / 384 /
   // 512 workgroups: 15.5 / 11.3 / 13.5 / 12.6), as far as every wave keeps a
-  // tile, the partials fit the static scratch and the merges its counters.
+  // tile, the partials fit the static scratch and the merges its counters.  Up to
+  // 256 keys, two tiles a wave, the merge costs more than the second tile where
+  // two workgroups share a CU (129 to 256 keys in two splits: 1.09 times as long in
+  // the median of 480 prompt launches, 1.22 from 128 groups on, 1.02 for single
+  // tokens; 257 to 384 keys 0.93), the second tile more in the wider forms (head_dim
+  // 224 and 256 0.85, 100 0.86).
   const int G = n_heads / n_kv_heads, cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const bool one = append && n_tokens == 1;
   const int dt = built_tiles(head_dim), kmax = start_pos + n_tokens;
@@ -788,9 +793,10 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   float* part = nullptr;
   size_t part_bytes = 0;
   decode_scratch(&ctr, &part, &part_bytes);
+  const bool paired = dt <= 8 && head_dim % 8 == 0;  // two workgroups a CU
   long want = (cus - 1 + groups_layer * n_launch_layers) / (groups_layer * n_launch_layers);
   if (ks != 4) want = 1;
-  want = std::min<long>({want, (kmax + 127) / 128, kGMaxSplit});
+  want = std::min<long>({want, paired && kmax <= 256 ? 1 : (kmax + 127) / 128, kGMaxSplit});
   a.split_len = ((kmax + (int)want - 1) / (int)want + 31) / 32 * 32;
   a.n_split = (kmax + a.split_len - 1) / a.split_len;
   const long groups = groups_layer * n_launch_layers;

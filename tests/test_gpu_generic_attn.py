@@ -39,6 +39,16 @@ def test_prefill_tiles(gpu, oracle_mod, case):
     TP.run_prefill(gpu, oracle_mod, cfg, start, n, seed=D + n)
 
 
+@pytest.mark.parametrize("keys", [128, 129, 256, 257, 385])
+@pytest.mark.parametrize("D", [80, 96])
+def test_key_splits(gpu, oracle_mod, D, keys):
+    """Launches of few workgroups split their keys from 257 on: one token and a
+    prompt that end at each edge."""
+    cfg = gpu.AttnConfig(2, 6, 2, D, keys, 1e4, 0)
+    TD.run_decode(gpu, oracle_mod, cfg, keys - 1, seed=keys)
+    TP.run_prefill(gpu, oracle_mod, cfg, keys - 20, 20, seed=keys)
+
+
 @pytest.mark.parametrize("D,n", [(66, 20), (72, 33), (80, 48), (96, 63), (112, 17), (120, 65)])
 def test_prefill_two_tiles_a_workgroup(gpu, oracle_mod, D, n):
     """From 4 x 256 column tiles in a launch a workgroup takes two of them:
