@@ -794,25 +794,35 @@ int g_prefill_ksplit = 0;
 // heads 11.5 -> 9.1, at start 1000 22.6 -> 17.0; 509 tokens at head_dim 128, 16
 // q and 8 kv heads 28.7 -> 24.7; one token after 8000 38 -> 17.  Launches of
 // more units than a quarter of the CUs lose (512 tokens of the first: 18.0 ->
-// 21.1), and so do long contexts, by wave tiles (32 keys, 16 columns) per CU:
-// above about 50 at head_dim 64 (128 tokens at start 8000: 55 -> 67 us) and 20
-// at 128 (200 tokens at start 1000: 29 -> 33), unless the unit's columns fill
-// one wave in four at most (2 tokens at start 8000, 22 layers: 125 -> 49; at
-// head_dim 128 two tiles then read each K/V row twice: 28 columns, 112 units 58 ->
-// 42, but 20 columns, 512 units 73 -> 80).
+// 21.1), and so do long contexts, by wave tiles (32 keys, 16 columns) per CU
+// (`most`): at head_dim 64 128 tokens at start 8000 (190) 55 -> 67, 157 at 1162 of 28
+// q and 4 kv heads (42) 23.6 -> 25.7; at 128, 551 at 768 of 4 heads (18, keys
+// split) 30.5 -> 32.7, but 740 of 8 heads (17, one workgroup a tile) 1.17 times
+// faster, unless of one or two kv heads of several layers (663 tokens, 4
+// layers, 13: 26.8 -> 28.6).  A unit whose columns fill one wave in four at most
+// pays for any context (2 tokens at start 8000, 22 layers: 125 -> 49); with two
+// column tiles each K/V row is read twice (28 columns, 112 units 58 -> 42, but
+// 20 columns, 512 units 73 -> 80).
+// A single token saves the append's launch: with up to 16 q heads per kv head
+// always (4151 shapes, none slower), with more as far as few tiles read the
+// rows again (one kv head, head_dim 64: 48 q heads, start 25352, 110 -> 19 us, 71 of
+// 32 layers, start 23276, 123 -> 162; head_dim 128: 48 of 32 layers, start 9387,
+// 77 -> 114).
 // Prompts within two key tiles take either way the same time.
 static bool few_tiles_pay(const PrefillArgs& a, int head_dim, int cus) {
   if (g_prefill_split || g_prefill_ksplit) return false;  // the units' own splits, by tuning
-  const long G = a.n_heads / a.n_kv_heads, cols = a.n_tokens * G;
+  const long cols = (long)a.n_tokens * (a.n_heads / a.n_kv_heads);
   const long key_tiles = (a.start_pos + a.n_tokens + kKT - 1) / kKT;
-  if (a.n_tokens == 1) return true;
-  if (key_tiles > 8 &&
-      (cols <= 16 || (cols <= 32 && (head_dim == 64 || (long)a.n_units * 2 <= cus))))
+  const bool one = a.n_tokens == 1, layers_of_few = a.n_launch_layers > 1 && a.n_kv_heads <= 2;
+  if ((one || key_tiles > 8) && (cols <= 16 || (cols <= 32 && (long)a.n_units * 2 <= cus)))
     return true;
-  const double tiles = (double)a.n_launch_layers * a.n_kv_heads * ((cols + 15) / 16) *
-                       (a.start_pos + 0.5 * a.n_tokens) / kKT;
-  return (long)a.n_units * 4 <= cus && key_tiles >= 3 &&
-         tiles <= (head_dim == 64 ? 48.0 : 20.0) * cus;
+  const long groups = (long)a.n_launch_layers * a.n_kv_heads * ((cols + 15) / 16);
+  const double tiles = groups * (a.start_pos + 0.5 * a.n_tokens) / kKT;
+  const double most = head_dim == 64 ? 40 : groups < cus ? 16 : layers_of_few ? 12 : 20;
+  if (one)
+    return groups * (head_dim == 64 ? 4 : 8) <= cus ||
+           (groups <= 2L * cus && tiles <= most * cus);
+  return (long)a.n_units * 4 <= cus && key_tiles >= 3 && tiles <= most * cus;
 }
 
 int plh::attn_prefill(int n_layers, int n_heads, int n_kv_heads, int head_dim, int max_seq_len,

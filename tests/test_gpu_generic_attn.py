@@ -128,6 +128,17 @@ def test_small_prefill_launches_match_units(gpu, case):
     assert_attn_close(got[0][0][:, :cfg.q_dim], got[1][0][:, :cfg.q_dim], D, what="few")
 
 
+@pytest.mark.parametrize("case", [  # layers, n_heads, n_kv_heads, head_dim, start
+    (1, 48, 1, 64, 300), (2, 71, 1, 128, 900), (3, 40, 2, 128, 70),  # 16-column tiles
+    (16, 96, 2, 128, 2100), (20, 71, 1, 64, 6000)])                   # units
+def test_one_token_wide_groups(gpu, oracle_mod, case):
+    """plh_attn_prefill of a single token with more than 16 q heads per kv head,
+    on either side of the rule for many tiles over long contexts."""
+    L, Hq, Hkv, D, start = case
+    cfg = gpu.AttnConfig(L, Hq, Hkv, D, start + 2, 1e4, 0)
+    TP.run_prefill(gpu, oracle_mod, cfg, start, 1, seed=start, check_layers=[0, L - 1])
+
+
 def test_prefill_later_rows_do_not_matter(gpu):
     """Tokens 0..19 give the same bits whatever finite rows tokens 20..39 hold;
     with infinities and NaNs among them (whose tiles are taken again in fp32)
