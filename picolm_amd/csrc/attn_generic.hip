@@ -54,6 +54,7 @@ namespace {
 
 constexpr int kGThreads = 256;
 constexpr int kGMaxD = 256;
+constexpr int kGChunk = kGThreads;  // generic_rows_kernel: positions, one per thread
 constexpr int kGSq = 8 * ((kGMaxD / 8 + 3) / 4 * 4 + 4);  // rms_sq_pitch(256) rows of 8
 constexpr int kGMaxSplit = 16;
 constexpr int kGCtrPitch = 32;  // counters on 128-byte lines of their own
@@ -694,13 +695,156 @@ generic_attn_kernel(GenericArgs a) {
   }
 }
 
-// d tiles for which two column tiles a workgroup are built (more don't fit LDS).
+// Maximum (MAX) or sum of v over the workgroup; every thread gets it.
+template <bool MAX>
+__device__ __forceinline__ float block_reduce(float v, float* wred) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float w = __shfl_xor(v, o);
+    v = MAX ? fmaxf(v, w) : v + w;
+  }
+  __syncthreads();  // the previous reduction's readers are done with wred
+  if ((threadIdx.x & 63) == 0) wred[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float r = wred[0];
+#pragma unroll
+  for (int i = 1; i < kGThreads / 64; ++i) r = MAX ? fmaxf(r, wred[i]) : r + wred[i];
+  return r;
+}
+
+// dot(q, k row) over D elements (q in LDS, the row fp16 bits in HBM): 16-byte
+// loads when D is a multiple of 8 (every row offset then is too), 4-byte ones
+// otherwise (D is even); four partial sums.
+__device__ __forceinline__ float row_dot(const float* qs, const uint16_t* kr, int D) {
+  float d4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (D % 8 == 0) {
+    const uint4* kp = (const uint4*)kr;
+    const int nw = D / 8;
+    for (int j = 0; j < nw; j += 4) {  // four 16-byte loads issued together
+      uint4 w[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) w[b] = j + b < nw ? kp[j + b] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const uint32_t ws[4] = {w[b].x, w[b].y, w[b].z, w[b].w};
+        const float* qq = qs + 8 * (j + b);
+        if (j + b < nw) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            d4[u] = d4[u] + qq[2 * u] * f16_bits_to_f32((uint16_t)(ws[u] & 0xFFFFu));
+            d4[u] = d4[u] + qq[2 * u + 1] * f16_bits_to_f32((uint16_t)(ws[u] >> 16));
+          }
+        }
+      }
+    }
+  } else {
+    const uint32_t* kp = (const uint32_t*)kr;
+    for (int j = 0; j < D / 2; ++j) {
+      const uint32_t w = kp[j];
+      float& d = d4[j & 3];
+      d = d + qs[2 * j] * f16_bits_to_f32((uint16_t)(w & 0xFFFFu));
+      d = d + qs[2 * j + 1] * f16_bits_to_f32((uint16_t)(w >> 16));
+    }
+  }
+  return (d4[0] + d4[1]) + (d4[2] + d4[3]);
+}
+
+// Few keys of a wide head (few_keys): one workgroup per (layer, token, q head) on
+// the VALU, after the append.  The positions in chunks of 256, one per thread:
+// scores, the chunk's maximum, exp weights and the rescaled sums of the online
+// softmax, v accumulated by one thread per d.
+__global__ __launch_bounds__(kGThreads) void generic_rows_kernel(GenericArgs a) {
+  __shared__ float qs[kGMaxD];
+  __shared__ float ps[kGChunk];
+  __shared__ __align__(16) float sq[kGSq];
+  __shared__ float red[8];
+  __shared__ float wred[kGThreads / 64];
+  const int tid = threadIdx.x;
+  const int D = a.D, kv_dim = a.n_kv_heads * D, G = a.n_heads / a.n_kv_heads;
+  const int h = blockIdx.x % a.n_heads;
+  const int t = (blockIdx.x / a.n_heads) % a.n_tokens;
+  const int li = blockIdx.x / (a.n_heads * a.n_tokens);
+  const int pos = a.start_pos + t, kvh = h / G;
+  const size_t row = (size_t)li * a.n_tokens + t;
+  load_normed(a.q + row * a.n_heads * D + (size_t)h * D, a.qn ? a.qn + (size_t)li * D : nullptr,
+              D, a.norm_eps, qs, sq, red);
+  const float* cr = a.cos_t + (size_t)pos * (D / 2);
+  const float* sr = a.sin_t + (size_t)pos * (D / 2);
+  for (int i = tid; i < D / 2; i += kGThreads) {
+    int i0, i1;
+    pair_of(a.rope_type, D, i, i0, i1);
+    float x0 = qs[i0], x1 = qs[i1];
+    rope_rotate(x0, x1, cr[i], sr[i]);
+    qs[i0] = x0;
+    qs[i1] = x1;
+  }
+  __syncthreads();
+  const size_t layer_off = (size_t)(a.layer0 + li) * a.max_seq_len * kv_dim + (size_t)kvh * D;
+  const uint16_t* kl = a.kc + layer_off;
+  const uint16_t* vl = a.vc + layer_off;
+  const float root = sqrtf((float)D);
+  float m = kNegBig, l = 0.0f, acc = 0.0f;  // acc: element d = tid of the output
+  for (int c0 = 0; c0 <= pos; c0 += kGChunk) {
+    const int p = c0 + tid;
+    float s = kNegBig;
+    if (p <= pos) s = row_dot(qs, kl + (size_t)p * kv_dim, D) / root;
+    const float mn = fmaxf(m, block_reduce<true>(s, wred));
+    const float e = p <= pos ? expf(s - mn) : 0.0f;
+    ps[tid] = e;
+    const float esum = block_reduce<false>(e, wred);  // its barriers publish ps
+    const float corr = expf(m - mn);
+    l = l * corr + esum;
+    if (tid < D) {
+      const int np = min(kGChunk, pos + 1 - c0);
+      const uint16_t* vp = vl + (size_t)c0 * kv_dim + tid;
+      // eight v loads in flight, four independent partial sums
+      float s4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      int j = 0;
+      for (; j + 8 <= np; j += 8) {
+        uint16_t vb[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) vb[u] = vp[(size_t)(j + u) * kv_dim];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s4[u & 3] = s4[u & 3] + ps[j + u] * f16_bits_to_f32(vb[u]);
+      }
+      for (; j < np; ++j) s4[0] = s4[0] + ps[j] * f16_bits_to_f32(vp[(size_t)j * kv_dim]);
+      acc = acc * corr + ((s4[0] + s4[1]) + (s4[2] + s4[3]));
+    }
+    m = mn;
+    __syncthreads();  // ps is rewritten by the next chunk
+  }
+  if (tid < D) a.out[row * a.out_stride + (size_t)h * D + tid] = acc / l;
+}
+
+// d tiles for which two column tiles a workgroup are built (from 10 on, 77 KB and
+// more of LDS, a second workgroup would no longer fit a CU).
 constexpr bool two_tiles(int dt) { return dt > 4 && dt <= 8; }
 
 // 16-wide tiles of d that head_dim runs on: the next built number.
 int built_tiles(int head_dim) {
   const int t = (head_dim + 15) / 16;
   return t <= 6 ? t : t <= 8 ? 8 : t <= 10 ? 10 : t <= 12 ? 12 : 16;
+}
+
+// Whether generic_rows_kernel is the faster one: few keys at head dims whose
+// tiles a CU holds once (10 d tiles and more; 4-byte loads from 5 on).  There a
+// launch costs 10 to 12 us however few the keys, and as much again where the
+// tiles exceed the CUs (head_dim 160, 12 layers of 32 kv heads, 64 q heads, 1 key:
+// 15.5 us, 10.9 here; 85 keys and 128 q heads 16.7, 25.6).  us, tiles / rows:
+// head_dim 256, one token of up to 256 heads, 1.10 in the median to 32 keys, 1.03 to
+// 64; prompts of 2 to 8 tokens 1.25 to 16 keys, 1.15 to 192; 192 from 2 tokens on
+// 1.1 to 32 keys; 100 (4-byte loads) 1.1 to 192; 160 1.05 to 16.
+bool few_keys(int n_layers, int n_heads, int n_kv_heads, int head_dim, int start_pos,
+              int n_tokens, int cus) {
+  const int dt = built_tiles(head_dim), keys = start_pos + n_tokens;
+  if (dt < 10 && (head_dim % 8 == 0 || dt < 5)) return false;
+  const long rows = (long)n_layers * n_tokens * n_heads;
+  const long cols = (long)n_tokens * (n_heads / n_kv_heads);
+  if ((long)n_layers * n_kv_heads * ((cols + 15) / 16) > cus)
+    return rows <= 6L * cus && rows * keys <= (dt >= 12 ? 256L : 128L) * cus;
+  if (n_tokens == 1) return dt == 16 && keys <= 64 && rows <= cus;
+  if (rows <= cus && keys <= 192 && (dt == 16 || dt < 10)) return true;
+  return keys <= (dt == 16 ? 128 : dt == 12 ? 32 : 16) && rows <= (dt >= 12 ? 4L : 1L) * cus;
 }
 
 template <int DT, int KS, bool ONE>
@@ -777,7 +921,9 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // tokens; 257 to 384 keys 0.93), the second tile more in the wider forms (head_dim
   // 224 and 256 0.85, 100 0.86).
   const int G = n_heads / n_kv_heads, cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  const bool one = append && n_tokens == 1;
+  const bool rows = few_keys(n_launch_layers, n_heads, n_kv_heads, head_dim, start_pos,
+                             n_tokens, cus);
+  const bool one = append && n_tokens == 1 && !rows;
   const int dt = built_tiles(head_dim), kmax = start_pos + n_tokens;
   const long tiles = (long)n_kv_heads * ((n_tokens * G + 15) / 16) * n_launch_layers;
   // Two column tiles a workgroup halve its fixed chain per column but give a
@@ -817,7 +963,8 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
   // Layers go in as many launches as that takes (each is independent); one
   // fits: n_split is 1 unless the launch has fewer groups than CUs.
   const long per_layer =
-      std::max<long>(groups_layer * a.n_split, (long)n_tokens * n_kv_heads);
+      rows ? (long)n_tokens * n_heads
+           : std::max<long>(groups_layer * a.n_split, (long)n_tokens * n_kv_heads);
   const int step = (int)std::min<long>(n_launch_layers, max_wg / per_layer);
   const size_t q_dim = (size_t)n_heads * head_dim, kv_dim = (size_t)n_kv_heads * head_dim;
   hipStream_t st = ctx().stream;
@@ -836,16 +983,20 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
     if (v_rows) b.v_rows = v_rows + rows_before * kv_dim;
     const long nl = b.n_launch_layers;
     if (append && !one) {
-      const long rows = nl * n_tokens * n_kv_heads;
+      const long kv_rows = nl * n_tokens * n_kv_heads;
       if (b.kn)
-        hipLaunchKernelGGL(generic_append_norm_kernel, dim3((unsigned)rows), dim3(kGThreads), 0,
+        hipLaunchKernelGGL(generic_append_norm_kernel, dim3((unsigned)kv_rows), dim3(kGThreads), 0,
                            st, b);
       else
         hipLaunchKernelGGL(generic_append_kernel, dim3((unsigned)(nl * n_tokens * a.n_chunk)),
                            dim3(kGThreads), 0, st, b);
       if (check_hip(hipGetLastError(), "generic_append_kernel")) return -1;
     }
-    launch_attn(b, one, ks, (unsigned)(nl * groups_layer * a.n_split), st);
+    if (rows)
+      hipLaunchKernelGGL(generic_rows_kernel, dim3((unsigned)(nl * per_layer)), dim3(kGThreads), 0,
+                         st, b);
+    else
+      launch_attn(b, one, ks, (unsigned)(nl * groups_layer * a.n_split), st);
     if (check_hip(hipGetLastError(), "generic_attn_kernel")) return -1;
   }
   return 0;

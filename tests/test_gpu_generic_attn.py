@@ -9,7 +9,9 @@ import numpy as np
 import pytest
 
 import test_gpu_decode as TD
+import test_gpu_decode_rows as TR
 import test_gpu_prefill as TP
+import test_gpu_qknorm as TQ
 from attn_check import assert_attn_close, filled_cache, normal_f32
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +34,7 @@ def test_decode_groups_and_splits(gpu, oracle_mod, heads, pos):
 @pytest.mark.parametrize("case", [  # n_heads, n_kv_heads, head_dim, start, n
     (4, 4, 20, 0, 16), (4, 4, 48, 0, 17), (14, 2, 80, 5, 33), (8, 2, 96, 700, 3),
     (6, 6, 112, 64, 65), (8, 8, 144, 0, 40), (2, 1, 176, 31, 50), (2, 2, 250, 0, 70),
+    (2, 2, 250, 60, 70), (2, 1, 256, 0, 150),
     (8, 8, 80, 1200, 20)])
 def test_prefill_tiles(gpu, oracle_mod, case):
     Hq, Hkv, D, start, n = case
@@ -47,6 +50,33 @@ def test_key_splits(gpu, oracle_mod, D, keys):
     cfg = gpu.AttnConfig(2, 6, 2, D, keys, 1e4, 0)
     TD.run_decode(gpu, oracle_mod, cfg, keys - 1, seed=keys)
     TP.run_prefill(gpu, oracle_mod, cfg, keys - 20, 20, seed=keys)
+
+
+@pytest.mark.parametrize("case", [  # layers, n_heads, n_kv_heads, head_dim, start, n: keys
+    (1, 4, 4, 256, 63, 1), (1, 4, 4, 256, 64, 1),          # 64 of one token, 65 tiles
+    (12, 32, 32, 160, 84, 1), (12, 32, 32, 160, 85, 1),    # 32768 with 384 rows, more
+    (6, 48, 48, 208, 226, 1), (6, 48, 48, 208, 227, 1),    # 65536 with 288, more
+    (1, 6, 2, 224, 172, 20), (1, 6, 2, 224, 173, 20),      # 192 of a prompt, 193
+    (3, 6, 2, 224, 108, 20), (3, 6, 2, 224, 109, 20),      # 128 with 360 rows, 129
+    (1, 8, 2, 192, 0, 32), (1, 8, 2, 192, 0, 33),          # 32, 33
+    (1, 8, 8, 100, 172, 20), (1, 8, 8, 100, 173, 20),      # 192 with 160 rows, 193
+    (1, 16, 2, 66, 0, 16), (1, 17, 1, 66, 0, 16),          # 256 rows, 272
+    (1, 8, 8, 160, 0, 16), (1, 8, 4, 160, 0, 17)])         # 16, 17
+def test_few_keys_of_wide_heads(gpu, oracle_mod, case):
+    """Either side of the rule that runs one workgroup per token and q head."""
+    L, Hq, Hkv, D, start, n = case
+    cfg = gpu.AttnConfig(L, Hq, Hkv, D, start + n + 1, 1e4, D // 4 % 2)
+    TP.run_prefill(gpu, oracle_mod, cfg, start, n, seed=start + n, check_layers=[0, L - 1])
+    if n == 1:
+        TD.run_decode(gpu, oracle_mod, cfg, start, seed=start, check_layers=[0, L - 1], poison=True)
+
+
+def test_few_keys_qknorm_and_rows(gpu, oracle_mod):
+    """The same with QK-norm, two prompt chunks and a token after them, and with
+    the appended rows mirrored."""
+    TQ.test_prefill_qknorm_chunks_then_decode(gpu, oracle_mod, (1, 6, 2, 256, 512, 1e4, 1))
+    TQ.test_decode_qknorm(gpu, oracle_mod, (2, 8, 4, 248, 64, 1e4, 0), 20)
+    TR.test_decode_rows_match_plain_decode(gpu, (2, 8, 2, 256, 300, 1, 0, 2, 20, True), False)
 
 
 @pytest.mark.parametrize("D,n", [(66, 20), (72, 33), (80, 48), (96, 63), (112, 17), (120, 65)])
