@@ -542,14 +542,25 @@ constexpr size_t kLds = 160 << 10;  // of a CU
 
 int cu_count() { return ctx().num_cus > 0 ? ctx().num_cus : 256; }
 
+// Whether the eight-wave form of a launch is built: its LDS fits a CU (a Q6_K
+// pair's exchanged terms don't).
+bool eight_built(int qtype, bool pair) {
+  if (!pair) return true;
+  return (qtype == kTypeQ4K   ? lds_bytes<Q4KM, 8, true>()
+          : qtype == kTypeQ6K ? lds_bytes<Q6KM, 8, true>()
+                              : lds_bytes<Q80M, 8, true>()) <= kLds;
+}
+static_assert(std::max({lds_bytes<Q4KM, 8, false>(), lds_bytes<Q6KM, 8, false>(),
+                        lds_bytes<Q80M, 8, false>()}) <= kLds, "plain launches: always built");
+
 // Eight waves on a row tile: where the launch's tiles leave CUs idle, two waves
 // a SIMD instead of one hide each other's MFMA and LDS waits; not for rows of
-// a chunk or two, and a Q6_K pair's exchanged terms don't fit the LDS.
+// a chunk or two.
 // Measured, us for 8 / 4 waves: n = 2048, 128 tiles, Q4_K 9.4 / 11.5, Q6_K 11.9 /
 // 13.7, Q8_0 12.0 / 14.5; n = 5632 20.1 / 27.9; n = 512 4.4 / 4.4 (Q6_K 5.7 / 5.4);
 // 384 tiles of n = 2048 17.6 / 15.7.
-bool eight_waves(const GemvArgs& a, long tiles, bool q6_pair) {
-  return tiles <= cu_count() && a.n >= 1024 && !q6_pair;
+bool eight_waves(const GemvArgs& a, long tiles, int qtype, bool pair) {
+  return tiles <= cu_count() && a.n >= 1024 && eight_built(qtype, pair);
 }
 
 // Waves per row tile, from the launch's 16 x 16 tiles (a pair's count once):
@@ -558,11 +569,11 @@ bool eight_waves(const GemvArgs& a, long tiles, bool q6_pair) {
 // 1408 35 / 32 / 37, 5632 114 / 95 / 94; Q6_K 256 13.6 / 21 / 28, 1024 36 /
 // 32 / 30, 5632 179 / 142 / 137.  Q8_0's products keep four tiles of
 // registers each and spill the unsplit form: 5632 tiles 179 / 156 / 213.
-int waves_per_tile(const GemvArgs& a, long tiles, bool q8, bool q6_pair) {
-  if (eight_waves(a, tiles, q6_pair)) return 8;
+int waves_per_tile(const GemvArgs& a, long tiles, int qtype, bool pair) {
+  if (eight_waves(a, tiles, qtype, pair)) return 8;
   const int cus = cu_count();
   if (tiles < 4L * cus) return 4;
-  return tiles < 8L * cus || q8 ? 2 : 1;
+  return tiles < 8L * cus || qtype == kTypeQ8_0 ? 2 : 1;
 }
 
 BatchShape shape_of(const GemvArgs& a, int n_tok, int x_stride, int out_stride, int kw) {
@@ -585,7 +596,7 @@ long tiles_of(const GemvArgs& a, int n_tok) {
 }
 
 template <class F, int KW>
-void launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
+int launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
   const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(64 * waves_of(KW));
   if (!pair) {
     hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, false>), grid, block, (lds_bytes<F, KW, false>()),
@@ -593,19 +604,20 @@ void launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st)
   } else if constexpr (lds_bytes<F, KW, true>() <= kLds) {
     hipLaunchKernelGGL((gemm_mfma_kernel<F, KW, true>), grid, block, (lds_bytes<F, KW, true>()),
                        st, a, b);
+  } else {
+    set_error("gemm_mfma: no pair of %d waves a tile", KW);
+    return -1;
   }
+  return check_hip(hipGetLastError(), "gemm_mfma_kernel launch");
 }
 template <class F>
-void launch_f(int kw, bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
-  if (kw == 8) {
-    launch_k<F, 8>(pair, a, b, st);
-  } else if (kw == 4) {
-    launch_k<F, 4>(pair, a, b, st);
-  } else if (F::kHalf || kw == 2) {  // Q8_0: waves_per_tile has no 1
-    launch_k<F, 2>(pair, a, b, st);
-  } else {
-    if constexpr (!F::kHalf) launch_k<F, 1>(pair, a, b, st);
+int launch_f(int kw, bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
+  if (kw == 8) return launch_k<F, 8>(pair, a, b, st);
+  if (kw == 4) return launch_k<F, 4>(pair, a, b, st);
+  if constexpr (!F::kHalf) {  // Q8_0: waves_per_tile has no 1
+    if (kw == 1) return launch_k<F, 1>(pair, a, b, st);
   }
+  return launch_k<F, 2>(pair, a, b, st);
 }
 
 template <int KW, bool Q8>
@@ -639,23 +651,18 @@ bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
   const long tiles = tiles_of(a, n_tok), cus = cu_count();
   const double more = (double)std::min((tiles - 1) / cus, 3L);  // tiles a CU past the first
   double unit = q4 ? 0.28 + 0.17 * more : q8 ? 0.375 + 0.23 * more : 0.35 + 0.27 * more;
-  if (eight_waves(a, tiles, pair && qtype == kTypeQ6K)) unit = q4 ? 0.21 : 0.29;
+  if (eight_waves(a, tiles, qtype, pair)) unit = q4 ? 0.21 : 0.29;
   const double chain = unit * ((a.n + 63) / 64) * (pair ? 2 : 1);
   return 2.8 + std::max(chain, work) < valu;
 }
 
 int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride) {
-  const int kw = waves_per_tile(a, tiles_of(a, n_tok), qtype == kTypeQ8_0,
-                                pair && qtype == kTypeQ6K);
+  const int kw = waves_per_tile(a, tiles_of(a, n_tok), qtype, pair);
   const BatchShape b = shape_of(a, n_tok, x_stride, out_stride, kw);
   hipStream_t st = ctx().stream;
-  if (qtype == kTypeQ4K)
-    launch_f<Q4KM>(kw, pair, a, b, st);
-  else if (qtype == kTypeQ8_0)
-    launch_f<Q80M>(kw, pair, a, b, st);
-  else
-    launch_f<Q6KM>(kw, pair, a, b, st);
-  return check_hip(hipGetLastError(), "gemm_mfma_kernel launch");
+  if (qtype == kTypeQ4K) return launch_f<Q4KM>(kw, pair, a, b, st);
+  if (qtype == kTypeQ8_0) return launch_f<Q80M>(kw, pair, a, b, st);
+  return launch_f<Q6KM>(kw, pair, a, b, st);
 }
 
 bool gemm_mfma_multi_takes(const int* qtype) {
@@ -669,7 +676,7 @@ int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride
   long tiles = 0;
   for (int i = 0; i < 3; ++i) tiles += tiles_of(a[i], n_tok);
   const bool q8 = qtype[0] == kTypeQ8_0;
-  const int kw = waves_per_tile(a[0], tiles, q8, false);
+  const int kw = waves_per_tile(a[0], tiles, qtype[0], false);
   for (int i = 0; i < 3; ++i) {
     m.seg[i] = a[i];
     m.qtype[i] = qtype[i];
