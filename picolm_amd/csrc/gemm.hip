@@ -595,6 +595,15 @@ long tiles_of(const GemvArgs& a, int n_tok) {
   return (long)((a.d + kMT - 1) / kMT) * ((n_tok + kMT - 1) / kMT);
 }
 
+// A launch holds fewer than 2^32 threads, here 2^32 / 256 workgroups of 512 outputs
+// (32 GiB) in the smallest case.  The VALU kernel's hold up to 2048 where rows
+// are short.
+bool launchable(int qtype, const GemvArgs& a, int n_tok, bool pair) {
+  const int kw = waves_per_tile(a, tiles_of(a, n_tok), qtype, pair);
+  const BatchShape b = shape_of(a, n_tok, 0, 0, kw);
+  return 8LL * ((b.row_tiles + 7) / 8) * b.tok_tiles * 64 * waves_of(kw) < 1LL << 32;
+}
+
 template <class F, int KW>
 int launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
   const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(64 * waves_of(KW));
@@ -642,6 +651,7 @@ namespace plh {
 // 128 tokens the two take 8.7 / 12.2 / 19 / 70 and 9.4 / 9.4 / 9.4 / 25 us; at 2304
 // x 6743 Q6_K and 2 tokens (two tiles a CU) 13.8 and 20.4.
 bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
+  if (!launchable(qtype, a, n_tok, pair)) return false;
   const double w = 1e-6 * a.n * (double)a.d * (pair ? 2 : 1);
   const bool q4 = qtype == kTypeQ4K, q8 = qtype == kTypeQ8_0;
   const double least = q4 ? (n_tok > 3 ? 11.5 : 8) : q8 ? (n_tok > 3 ? 8 : 6) : n_tok > 2 ? 12 : 10;

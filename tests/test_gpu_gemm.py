@@ -89,6 +89,28 @@ def test_matmul_batch_special_values(gpu, oracle_mod, qtype):
     W.free()
 
 
+def test_matmul_batch_more_outputs_than_a_launch(gpu, oracle_mod):
+    """131072 rows of one block and 65600 tokens: 2^33 outputs and some, past
+    what one launch of 16 x 16 tiles can hold (2^32 threads), not past the VALU
+    kernel's.  Some tokens' rows bit for bit, the last ones among them."""
+    P, O = gpu, oracle_mod
+    n, d, tokens = 32, 131072, 65600
+    rng = np.random.default_rng(33)
+    rows = S.random_weights(rng, Q8, n, d, S.unit_scale_exp(Q8, n))
+    W = G.QMatrix(Q8, n, d, rows)
+    X = rng.standard_normal((tokens, n)).astype(np.float32)
+    dx, out = P.DeviceBuffer.from_numpy(X), P.DeviceBuffer(4 * tokens * d)
+    P.check(P.lib.plh_matmul_batch(Q8, n, d, C.c_void_p(W.ptr), C.c_void_p(dx.ptr), tokens,
+                                   C.c_void_p(out.ptr)), "plh_matmul_batch")
+    got = np.empty(d, np.float32)
+    for t in (0, 40000, 65535, 65536, tokens - 1):
+        P.check(P.lib.plh_memcpy_dtoh(got.ctypes.data, out.ptr + 4 * t * d, 4 * d), "dtoh")
+        assert_bits(got, O.matmul(rows, X[t], n, d, Q8), t)
+    for b in (dx, out):
+        b.free()
+    W.free()
+
+
 def layer0_rows_exact(P, O, n_tok, **kw):
     """A prompt's layer-0 cached rows (exact order, nothing transcendental)
     against the oracle's, bit for bit."""
