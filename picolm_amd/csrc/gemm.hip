@@ -11,7 +11,7 @@
 // from zero.  v_mfma_f32_16x16x1_4b_f32 (four independent 16 x 16 tiles, one
 // step each) forms four of a Q6_K group's running sums in two steps, or the
 // four rounded products of a Q8_0 block's lane.  A weight is then converted
-// to fp32 once per 16 or 32 tokens instead of once per token, and only the
+// to fp32 once per 16 tokens instead of once per token, and only the
 // adds between the running sums, the scales and the block chain stay on the
 // VALU.
 //
@@ -27,6 +27,7 @@
 // against 130: the vector memory path handles the 16 tokens' lines one by
 // one); two token tiles a wave (88 against 94 us on that shape, slower below it).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "gemv_formats.h"
@@ -604,6 +605,59 @@ bool launchable(int qtype, const GemvArgs& a, int n_tok, bool pair) {
   return 8LL * ((b.row_tiles + 7) / 8) * b.tok_tiles * 64 * waves_of(kw) < 1LL << 32;
 }
 
+// Which of the two batched kernels runs, by estimates in us fitted to both (34000 shapes
+// of n 64 to 11000, d 64 to 12000, 2 to 256 tokens, warm) so that the choice is
+// right rather than the estimate.  The VALU kernel: its latency, or its work per
+// weight, token and group of four tokens, of which a workgroup's idle lanes (169
+// units leave 87 of 256) waste a share.  Here: a wave's chain of units, longer with
+// every further tile a CU (its workgroups share the SIMDs; from four on fewer waves
+// share a tile), or, with the chip full, the work of the padded token tiles.
+// VALU / here: 2048 x 2048 Q4_K, 2 / 4 / 16 / 128 tokens 8.7 / 12.2 / 19 / 70 and
+// 9.4 / 9.4 / 9.4 / 25; Q8_0 5408 x 1581, 39 tokens 75 and 47; Q6_K 512 x 9343, 2
+// tokens 7.7 and 10.8; the pair 2816 x 7936 Q4_K, 5 tokens 55 and 28.  Of these 33
+// shapes run more than 2% longer than on the VALU kernel, 484 more than 10%
+// longer than on the better one; of 8800 pairs 69 and (5%) 261.
+struct Rule {
+  double least[3], least_n;    // VALU latency: 2, 3, more tokens; per unit of a row
+  double valu0, valu1, valu4;  // a launch; 10^6 weights times tokens, times fours
+  double lanes;                // its power of the active lanes' share
+  double mfma0, unit[5];       // here: a launch; units by tiles a CU (1, 2, 3, more;
+  double work;                 // eight waves); 10^6 weights times padded tokens
+  double pair;                 // a pair's chain and work
+};
+constexpr Rule kRule4K = {{8.8, 10.1, 12.4}, 0.0111, 7.3, 0.107, 0.0476, 0.74,
+                          3.34, {0.283, 0.302, 0.4065, 0.614, 0.191}, 0.0508, 1.8};
+constexpr Rule kRule6K = {{7.34, 8.2, 12.8}, 0.1, 7.16, 0.165, 0.107, 0.51,
+                          3.713, {0.2958, 0.4896, 0.7191, 1.193, 0.2479}, 0.038, 1};
+constexpr Rule kPair6K = {{10, 12, 12}, 0, 8, 0.22, 0, 0,
+                          2.8, {0.35, 0.62, 0.89, 1.16, 0}, 0.046, 2};  // no eight waves
+constexpr Rule kRule80 = {{5.77, 6.94, 7.58}, 0.0308, 5.79, 0.086, 0.169, 1.04,
+                          3.47, {0.317, 0.538, 0.695, 0.908, 0.278}, 0.0569, 2.1};
+
+const Rule& rule_of(int qtype, bool pair) {
+  if (qtype == kTypeQ6K) return pair ? kPair6K : kRule6K;
+  return qtype == kTypeQ4K ? kRule4K : kRule80;
+}
+
+int units64(const GemvArgs& a) { return (a.n + 63) / 64; }
+double mega(const GemvArgs& a) { return 1e-6 * a.n * (double)a.d; }
+
+double valu_us(int qtype, const GemvArgs& a, int n_tok, bool pair) {
+  const Rule& r = rule_of(qtype, pair);
+  const double lanes = (double)a.units * a.row_par / (a.unit_iters * (double)kThreads);
+  const double work = mega(a) * (r.valu1 * n_tok + r.valu4 * ((n_tok + 3) / 4));
+  return std::max(r.least[n_tok > 3 ? 2 : n_tok > 2] + r.least_n * units64(a),
+                  r.valu0 + (pair ? 2 : 1) * work / std::pow(lanes, r.lanes));
+}
+// of a launch of so many tiles
+double unit_us(int qtype, const GemvArgs& a, long tiles, bool pair) {
+  const long past_first = std::min((tiles - 1) / cu_count(), 3L);
+  return rule_of(qtype, pair).unit[eight_waves(a, tiles, qtype, pair) ? 4 : past_first];
+}
+double work_us(int qtype, const GemvArgs& a, int n_tok, bool pair) {
+  return rule_of(qtype, pair).work * mega(a) * ((n_tok + kMT - 1) / kMT * kMT);
+}
+
 template <class F, int KW>
 int launch_k(bool pair, const GemvArgs& a, const BatchShape& b, hipStream_t st) {
   const dim3 grid(grid_of(b.row_tiles, b.tok_tiles)), block(64 * waves_of(KW));
@@ -642,28 +696,12 @@ void launch_multi(const MultiBatch& m, hipStream_t st) {
 
 namespace plh {
 
-// The estimates, in us, are fits to measured times of both kernels (n 256 to
-// 11008, d 65 to 11264, 2 to 128 tokens, warm): the VALU kernel's latency (a group
-// of four tokens takes longer than two) or its work per weight and token; here
-// a wave's chain of units, longer with every further tile a CU (its workgroups
-// share the SIMDs; from four a CU on fewer waves share a tile), or, with the chip
-// full, the work of the padded token tiles.  At 2048 x 2048 Q4_K and 2 / 4 / 16 /
-// 128 tokens the two take 8.7 / 12.2 / 19 / 70 and 9.4 / 9.4 / 9.4 / 25 us; at 2304
-// x 6743 Q6_K and 2 tokens (two tiles a CU) 13.8 and 20.4.
 bool gemm_mfma_pays(int qtype, const GemvArgs& a, int n_tok, bool pair) {
   if (!launchable(qtype, a, n_tok, pair)) return false;
-  const double w = 1e-6 * a.n * (double)a.d * (pair ? 2 : 1);
-  const bool q4 = qtype == kTypeQ4K, q8 = qtype == kTypeQ8_0;
-  const double least = q4 ? (n_tok > 3 ? 11.5 : 8) : q8 ? (n_tok > 3 ? 8 : 6) : n_tok > 2 ? 12 : 10;
-  const double valu =
-      std::max(least, (q8 ? 6.0 : 8.0) + w * n_tok * (q4 ? 0.12 : q8 ? 0.125 : 0.22));
-  const double work = w * ((n_tok + kMT - 1) / kMT * kMT) * (q4 ? 0.032 : q8 ? 0.053 : 0.046);
-  const long tiles = tiles_of(a, n_tok), cus = cu_count();
-  const double more = (double)std::min((tiles - 1) / cus, 3L);  // tiles a CU past the first
-  double unit = q4 ? 0.28 + 0.17 * more : q8 ? 0.375 + 0.23 * more : 0.35 + 0.27 * more;
-  if (eight_waves(a, tiles, qtype, pair)) unit = q4 ? 0.21 : 0.29;
-  const double chain = unit * ((a.n + 63) / 64) * (pair ? 2 : 1);
-  return 2.8 + std::max(chain, work) < valu;
+  const Rule& r = rule_of(qtype, pair);
+  const double chain = unit_us(qtype, a, tiles_of(a, n_tok), pair) * units64(a);
+  return r.mfma0 + (pair ? r.pair : 1) * std::max(chain, work_us(qtype, a, n_tok, pair)) <
+         valu_us(qtype, a, n_tok, pair);
 }
 
 int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride) {
@@ -675,9 +713,24 @@ int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, 
   return launch_f<Q6KM>(kw, pair, a, b, st);
 }
 
-bool gemm_mfma_multi_takes(const int* qtype) {
+// Nearly always: one launch beats three of the matrix cores, which small
+// matrices leave idle, and three of the VALU kernel but for two or three tokens of long
+// rows (Q8_0 n = 4096, 4096 + 2 x 512 rows: 34 us against 26; 128 tokens of
+// TinyLlama's 2048 + 2 x 256: 34 against 102).  Of 6950 shapes 12 lose more than 2%.
+bool gemm_mfma_multi_pays(const int* qtype, const GemvArgs* a, int n_tok) {
   const int q8 = (qtype[0] == kTypeQ8_0) + (qtype[1] == kTypeQ8_0) + (qtype[2] == kTypeQ8_0);
-  return q8 == 0 || q8 == 3;
+  if (q8 != 0 && q8 != 3) return false;
+  long tiles = 0, threads = 0;
+  for (int i = 0; i < 3; ++i) tiles += tiles_of(a[i], n_tok);
+  double apart = 0, first = 0, unit = 0, work = 0;
+  for (int i = 0; i < 3; ++i) {
+    apart += valu_us(qtype[i], a[i], n_tok, false);
+    first = std::max(first, rule_of(qtype[i], false).mfma0);
+    unit += unit_us(qtype[i], a[i], tiles, false) * tiles_of(a[i], n_tok) / tiles;
+    work += work_us(qtype[i], a[i], n_tok, false);
+    threads += tiles_of(a[i], n_tok) * 512;  // at most, but for the last tiles
+  }
+  return threads < 1LL << 31 && first + std::max(unit * units64(a[0]), work) < apart;
 }
 
 int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride,

@@ -1651,9 +1651,7 @@ int gemv_batch3_launch(const GemvCall* g) {
     together = together && g[s].n_tok > 1;
     if (g[s].n_tok > 1 && !batch_rb(a[s], false)) return -1;
   }
-  // one launch where the matrix cores would run the largest of the three
-  if (!together || !gemm_mfma_multi_takes(qtype) ||
-      !gemm_mfma_pays(qtype[0], a[0], g[0].n_tok, false)) {
+  if (!together || !gemm_mfma_multi_pays(qtype, a, g[0].n_tok)) {
     for (int s = 0; s < 3; ++s)
       if (gemv_launch(g[s])) return -1;
     return 0;

@@ -96,9 +96,9 @@ struct BatchShape {
 // gemm.hip: the batched GEMV on the matrix cores, x rows x_stride apart, out
 // rows (and gate, resid) out_stride apart; pair: gate a.w, up a.w2.  0 or -1.
 int gemm_mfma(int qtype, bool pair, const GemvArgs& a, int n_tok, int x_stride, int out_stride);
-// Three matrices over the same x in one launch: takes K quants only or Q8_0
-// only.
-bool gemm_mfma_multi_takes(const int* qtype);
+// Three matrices over the same x in one launch, K quants only or Q8_0 only, and
+// whether that is faster than three launches.
+bool gemm_mfma_multi_pays(const int* qtype, const GemvArgs* a, int n_tok);
 int gemm_mfma_multi(const int* qtype, const GemvArgs* a, int n_tok, int x_stride,
                     const int* out_stride);
 // Whether it is the faster of the two batched kernels for this shape.
