@@ -11,7 +11,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from attn_check import FWD_TOL_FAST
+from attn_check import FWD_TOL_FAST, KV_TOL
 from picolm_amd import gemv as G
 from picolm_amd import synth as S
 
@@ -166,3 +166,48 @@ def test_prompt_long_rows_few_tiles(gpu, oracle_mod, n_embd, gate, n_tok):
             assert np.array_equal(a, b)
     finally:
         dm.free()
+
+
+def prompt_rows_two_layers(P, O, n_tok, **kw):
+    """A prompt's cached rows against the oracle's: layer 0's bit for bit (exact
+    order), layer 1's, which every token's q, attention, o, gate/up pair and
+    down products of layer 0 reach, within one fp16 step and KV_TOL (silu's
+    expf and the softmax round apart)."""
+    cfg = dict(n_layers=2, vocab_size=64, max_seq_len=n_tok + 1, rope_type=0, rope_base=1e4,
+               eps=1e-5, **kw)
+    h = S.SynthModel(**cfg, seed=cfg["n_ffn"] + n_tok)
+    dm, orc = P.DeviceModel(h), O.OracleForward(h)
+    toks = np.arange(n_tok, dtype=np.int32) * 7 % 64
+    try:
+        dm.prefill(toks, 0)
+        P.synchronize()
+        orc.prefill(toks, 0, n_threads=8)
+        for a, b in zip(dm.fetch_cache(), (orc.kc, orc.vc)):
+            half = a.size // 2
+            assert np.array_equal(a[:half], b[:half])
+            x, y = O.f16_to_f32(a[half:]), O.f16_to_f32(b[half:])
+            step = np.spacing(np.maximum(np.abs(x), np.abs(y)).astype(np.float16))
+            bad = np.abs(x - y) > step.astype(np.float32) + KV_TOL * np.max(np.abs(y))
+            assert not bad.any(), np.flatnonzero(bad)[:8]
+    finally:
+        dm.free()
+
+
+@pytest.mark.parametrize("gate", [Q4, Q6, Q8])
+@pytest.mark.parametrize("n_ffn", [2080, 4128])
+def test_prompt_pair_many_tiles(gpu, oracle_mod, gate, n_ffn):
+    """The gate/up pair from 4 x 256 tiles (two waves a row tile) and, K quants,
+    from 8 x 256 (one wave, the last workgroup's rows half there)."""
+    types = dict(embd=Q8, output=Q8, q=Q8, k=Q8, v=Q8, o=Q8, gate=gate, up=gate, down=Q8)
+    prompt_rows_two_layers(gpu, oracle_mod, 120, n_embd=256, n_ffn=n_ffn, n_heads=4,
+                           n_kv_heads=2, head_dim=64, types=types)
+
+
+@pytest.mark.parametrize("q,k,v", [(Q4, Q4, Q6), (Q6, Q4, Q4), (Q8, Q8, Q8)])
+@pytest.mark.parametrize("n_embd,heads,n_tok", [(256, 42, 120), (256, 84, 119), (1024, 6, 17)])
+def test_prompt_qkv_waves(gpu, oracle_mod, q, k, v, n_embd, heads, n_tok):
+    """The joint q/k/v launch with two, one (Q8_0 two) and eight waves a row
+    tile; k's and v's rows end inside a workgroup's."""
+    types = dict(embd=Q8, output=Q8, q=q, k=k, v=v, o=Q8, gate=Q8, up=Q8, down=Q8)
+    prompt_rows_two_layers(gpu, oracle_mod, n_tok, n_embd=n_embd, n_ffn=128, n_heads=heads,
+                           n_kv_heads=3, head_dim=48, types=types)

@@ -87,6 +87,34 @@ def test_prefill_two_tiles_a_workgroup(gpu, oracle_mod, D, n):
     TP.run_prefill(gpu, oracle_mod, cfg, 0, n, seed=D + n, check_layers=[0, 10])
 
 
+@pytest.mark.parametrize("D,n,rope", [(80, 33, 0), (112, 49, 1)])
+def test_two_tiles_a_workgroup_qknorm(gpu, oracle_mod, D, n, rope):
+    """The same with QK-norm: the first and the last layer's outputs and rows."""
+    P, O = gpu, oracle_mod
+    L, H, S = 11, 48, n + 4
+    cfg = P.AttnConfig(L, H, H, D, S, 1e4, rope)
+    rng = np.random.default_rng(D + n)
+    q, k, v = (normal_f32(rng, (L, n, H * D), 3.0) for _ in "qkv")
+    qw, kw = (rng.uniform(0.5, 1.5, (L, D)).astype(np.float32) for _ in "qk")
+    d = [P.DeviceBuffer.from_numpy(x) for x in (q, k, v, qw, kw)]
+    cache, out = P.KVCache(cfg), P.DeviceBuffer(4 * L * n * H * D)
+    P.prefill(cache, 0, 0, n, d[0].ptr, d[1].ptr, d[2].ptr, out.ptr, None, L, q_norm=d[3].ptr,
+              k_norm=d[4].ptr, norm_eps=1e-5)
+    P.synchronize()
+    got = out.download(np.float32, (L, n, H * D))
+    rows = [c.reshape(L, S, H * D) for c in cache.fetch()]
+    cache.free()
+    shp = O.Shape(L, H, H, D, S, 1e4, rope)
+    cos_t, sin_t = O.rope_tables(S, D, 1e4)
+    want = [np.zeros(cfg.cache_elems, np.uint16) for _ in "kv"]
+    for l in (0, L - 1):
+        ref = O.attn_prefill(shp, l, 0, n, q[l].copy(), k[l].copy(), v[l], *want, cos_t, sin_t,
+                             q_norm=qw[l], k_norm=kw[l], eps=1e-5)
+        assert_attn_close(got[l], ref, D, what=f"two tiles, QK-norm, layer {l}")
+        for a, b in zip(rows, want):
+            assert np.array_equal(a[l], b.reshape(L, S, H * D)[l])
+
+
 def test_decode_unaligned_caches(gpu):
     """Caches that start 2 elements past a 16-byte boundary (4-byte loads): the
     same bits as aligned ones."""

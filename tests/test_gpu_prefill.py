@@ -123,9 +123,9 @@ SMALL = [
 
 
 # launches whose heavy q blocks are split into chunks of tiles (partials merged
-# afterwards): automatic for one-layer launches with few q blocks (a prompt
-# chunk late in the prompt), forced here through plh_set_tuning key 5 for the
-# other chunk sizes
+# afterwards): automatic for one-layer launches with few q blocks and too much
+# work for the 16-column tiles (a prompt chunk late in a long prompt), forced
+# here through plh_set_tuning key 5 for the other chunk sizes
 SPLIT = [
     # (n_layers, n_heads, n_kv_heads, head_dim, max_seq_len, theta, rope_type, start, n,
     #  layer, chunk tiles: 0 = automatic)
@@ -133,8 +133,11 @@ SPLIT = [
     (2, 32, 4, 64, 1024, 1e4, 0, 300, 333, 0, 2),   # prefix rows, ragged last block
     (2, 32, 8, 64, 800, 5e5, 0, 17, 700, 1, 16),    # Llama-3.2 heads
     (2, 32, 32, 128, 1100, 1e4, 0, 0, 1024, 0, 8),  # Llama-2 MHA, D = 128
-    (2, 8, 2, 128, 700, 1e6, 1, 40, 600, 1, 0),     # QWEN rotation, D = 128 (automatic)
-    (2, 32, 4, 64, 1200, 1e4, 0, 1024, 128, 1, 0),  # a 128-token chunk late in the prompt
+    (2, 8, 2, 128, 700, 1e6, 1, 40, 600, 1, 0),     # QWEN rotation, D = 128 (16-column tiles)
+    (2, 32, 4, 64, 1200, 1e4, 0, 1024, 128, 1, 0),  # a 128-token chunk late in the prompt (same)
+    (2, 8, 2, 128, 1400, 1e6, 1, 900, 400, 1, 0),   # automatic chunks of 4 tiles
+    (2, 8, 2, 128, 2200, 1e6, 1, 1600, 500, 1, 0),  # automatic chunks of 8
+    (1, 32, 4, 64, 6200, 1e4, 0, 6000, 128, 0, 0),  # the same at D = 64
 ]
 
 
@@ -150,11 +153,17 @@ def test_prefill_one_layer_split(gpu, oracle_mod, case):
         gpu.lib.plh_set_tuning(5, 0)
 
 
+@pytest.mark.parametrize("key5", [0, -1])
 @pytest.mark.parametrize("case", SMALL)
-def test_prefill_small(gpu, oracle_mod, case):
+def test_prefill_small(gpu, oracle_mod, case, key5):
+    """As the launch chooses (most on 16-column tiles) and on the units."""
     L, Hq, Hkv, D, S, theta, rt, start, n = case
     cfg = gpu.AttnConfig(L, Hq, Hkv, D, S, theta, rt)
-    run_prefill(gpu, oracle_mod, cfg, start, n, seed=start * 7 + n + D)
+    gpu.check(gpu.lib.plh_set_tuning(5, key5), "plh_set_tuning")
+    try:
+        run_prefill(gpu, oracle_mod, cfg, start, n, seed=start * 7 + n + D)
+    finally:
+        gpu.lib.plh_set_tuning(5, 0)
 
 
 # K-split workgroups (2 or 3 groups of 4 waves share a q block's tiles and
