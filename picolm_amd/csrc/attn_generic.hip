@@ -16,7 +16,9 @@
 //     v_mfma_f32_16x16x32_f16 with fp32 sums: K and V are fp16 already, and q
 //     (scaled by a power of two per column) and the weights go in as three
 //     fp16 parts, the lower ones scaled up (split3): all 24 bits of weights and
-//     q elements down to 2^-36 of the column's largest.  S = K q^T with the K rows
+//     q elements down to 2^-36 of the column's largest.  q's QK-norm sums over a
+//     column's 16 lanes (not the reference's AVX2 order, which only the cached k
+//     rows need).  S = K q^T with the K rows
 //     straight from the cache, O^T += V^T P^T with V^T through a wave's own
 //     LDS tile and ds_read_b64_tr_b16.  The S accumulators hold keys 4 g + v
 //     and 16 + 4 g + v of column c in lane (g, c), which is the PV operand if
@@ -25,10 +27,12 @@
 //     last to finish merges their partials.  Decode (one token) appends in the
 //     same launch: the workgroup whose range holds row pos rotates and rounds
 //     it and takes it from LDS.
-// generic_append_kernel, generic_append_norm_kernel  the prompt's rows: RoPE
+// generic_rows_kernel  few keys of wide heads (few_keys): a workgroup per (layer,
+//     token, q head) on the VALU.
+// generic_append_kernel, generic_append_rows_kernel  the rows, elsewhere: RoPE
 //     with the reference's four-product rotation and its fp16 rounding, a
-//     thread per rope pair; with QK-norm one workgroup per row (rmsnorm in the
-//     reference's AVX2 order).
+//     thread per rope pair; with QK-norm (rmsnorm in the reference's AVX2 order),
+//     and for a single token, one workgroup per row.
 // Cache rows are bit-identical to the reference's (and optionally mirrored
 // into caller row buffers); the softmax is exp2-based and per tile, so outputs
 // agree with the reference's within the attention tolerance.
@@ -129,7 +133,7 @@ __global__ __launch_bounds__(kGThreads) void generic_append_kernel(GenericArgs a
   }
 }
 
-__global__ __launch_bounds__(kGThreads) void generic_append_norm_kernel(GenericArgs a) {
+__global__ __launch_bounds__(kGThreads) void generic_append_rows_kernel(GenericArgs a) {
   __shared__ __align__(16) float sq[kGSq];
   __shared__ float red[8];
   __shared__ float kr[kGMaxD];
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(kGThreads) void generic_append_norm_kernel(GenericA
   const int li = blockIdx.x / (a.n_kv_heads * a.n_tokens);
   const int pos = a.start_pos + t;
   const size_t src = ((size_t)li * a.n_tokens + t) * kv_dim + (size_t)kvh * D;
-  load_normed(a.k + src, a.kn + (size_t)li * D, D, a.norm_eps, kr, sq, red);
+  load_normed(a.k + src, a.kn ? a.kn + (size_t)li * D : nullptr, D, a.norm_eps, kr, sq, red);
   const float* cr = a.cos_t + (size_t)pos * (D / 2);
   const float* sr = a.sin_t + (size_t)pos * (D / 2);
   const size_t dst =
@@ -984,8 +988,10 @@ int attn_generic(int n_heads, int n_kv_heads, int head_dim, int max_seq_len, int
     const long nl = b.n_launch_layers;
     if (append && !one) {
       const long kv_rows = nl * n_tokens * n_kv_heads;
-      if (b.kn)
-        hipLaunchKernelGGL(generic_append_norm_kernel, dim3((unsigned)kv_rows), dim3(kGThreads), 0,
+      // a token's few rows: a workgroup each (head_dim 256, 32 heads, with the
+      // attention: 10.9 us with a thread per rope pair, 9.6 so)
+      if (b.kn || n_tokens == 1)
+        hipLaunchKernelGGL(generic_append_rows_kernel, dim3((unsigned)kv_rows), dim3(kGThreads), 0,
                            st, b);
       else
         hipLaunchKernelGGL(generic_append_kernel, dim3((unsigned)(nl * n_tokens * a.n_chunk)),
