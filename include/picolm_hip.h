@@ -169,8 +169,13 @@ int plh_attn_decode_rows(int n_layers, int n_heads, int n_kv_heads, int head_dim
  * workspace.  It calls no hipMalloc / hipFree.  Returns -1 with a message
  * when a launch's partials would exceed the 16 MiB (very wide models: the
  * partials take n_units * min(G,16) * (head_dim+2) * 4 bytes, a few MiB at
- * the usual shapes).  Every call on a GPU shares that one array: calls that
- * overlap on one GPU race (the library's own stream serialises its calls). */
+ * the usual shapes); at head dims other than 64 and 128 the keys are then not
+ * split instead, and there are no partials.
+ * The array (arrival counters, zero between launches, and partials) also serves
+ * every decode and prefill launch of head dims other than 64 and 128,
+ * plh_forward's included, and the small plh_attn_prefill launches of these
+ * two.  All of these on a GPU share it: any that overlap race (the library's
+ * own stream serialises its calls). */
 int plh_attn_decode_noalloc(int n_layers, int n_heads, int n_kv_heads, int head_dim,
                             int max_seq_len, int rope_type, int layer0,
                             int n_launch_layers, int pos, const float *q,
@@ -191,7 +196,9 @@ int plh_attn_decode_noalloc(int n_layers, int n_heads, int n_kv_heads, int head_
  * rows 0..start_pos+bi, the prefix rows coming from the cache as the
  * reference's kvcache_load leaves them.  out_stride is a multiple of 4 and at
  * least n_heads*head_dim (the reference uses n_embd).  n_tokens = 0 is a
- * no-op. */
+ * no-op.  Small launches run on another kernel than plh_forward_prefill's
+ * attention of the same rows: the appended rows are the same bits, the outputs
+ * may differ in the last ones. */
 int plh_attn_prefill(int n_layers, int n_heads, int n_kv_heads, int head_dim,
                      int max_seq_len, int rope_type, int layer0,
                      int n_launch_layers, int start_pos, int n_tokens,
@@ -359,12 +366,14 @@ int plh_forward_prefill(const plh_model *m, const int *tokens, int n_tokens, int
  * launch of its own (1) instead of inside the GEMVs that read it (0,
  * default); key 5: prefill launches with fewer q blocks than workgroup slots
  * split their heavy blocks into chunks of tiles merged afterwards (0
- * automatic, small launches on 16-column tiles instead, -1 never, 2, 4, 8 or 16 tiles per chunk); key 6: prefill
+ * automatic, -1 never, 2, 4, 8 or 16 tiles per chunk); key 6: prefill
  * launches of at most one q block per CU run each block in a workgroup of 2
  * or 3 groups of 4 waves that share its tiles and merge in LDS (0
- * automatic, -1 never, 2 or 3 groups; head_dim 128 takes at most 2); key
- * 7: decode kernel (0 by shape, 1 split + combine, 2 stream-K with the merge
- * in the launch); key 8: stream-K workgroups (0 = by shape); key 9:
+ * automatic, -1 never, 2 or 3 groups; head_dim 128 takes at most 2); small
+ * plh_attn_prefill launches, single tokens among them, run on 16-column tiles
+ * instead of q blocks only while keys 5 and 6 are both 0; key 7: decode
+ * kernel (0 by shape, 1 split + combine, 2 stream-K with the merge in the
+ * launch); key 8: stream-K workgroups (0 = by shape); key 9:
  * stream-K tiles in flight per wave (0 = default, 2, 3, 4); key 10: the
  * single-vector weight GEMVs (plh_gemv*, gpu_try_matmul, plh_forward) keep
  * the reference's x86 AVX2 summation order bit for bit (1) or use the

@@ -58,18 +58,20 @@
 
 using namespace plh;
 
-// ---- static scratch of the allocation-free entry point ---------------------
-// plh_attn_decode_noalloc keeps its split partials in this file-scope device
-// array instead of the library workspace: each GPU holds its own copy until
-// the process ends, and every call on a GPU shares it (concurrent calls on one
-// GPU would race; the library's single stream serialises its own calls).  No
-// part of it needs clearing: every partial a launch reads was written by the
-// same launch.  In host code `scratch` is a host-side stand-in, not a device
+// ---- static scratch ---------------------------------------------------------
+// plh_attn_decode_noalloc and the 16-column kernel (attn_generic.hip, through
+// decode_scratch) keep their split partials and arrival counters in this
+// file-scope device array instead of the library workspace: each GPU holds its
+// own copy until the process ends, and every such launch on a GPU shares it
+// (launches that overlap would race; the library's single stream serialises its
+// calls).  The counters are zeroed once and every launch leaves them zero; the
+// partials need no clearing: every one a launch reads was written by the same
+// launch.  In host code `scratch` is a host-side stand-in, not a device
 // address: decode_scratch_setup (called by plh_init with the device current)
 // looks the device address up once per device, and launches use that.
 static constexpr size_t kScratchBytes = 16u << 20;
-// its first kScratchCounterBytes hold the stream-K kernel's arrival counters,
-// the rest the split partials
+// its first kScratchCounterBytes hold the arrival counters, the rest the split
+// partials
 static constexpr size_t kScratchCounterBytes = (size_t)kDecodeCounters * sizeof(unsigned);
 static constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];

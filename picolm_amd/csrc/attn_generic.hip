@@ -41,11 +41,12 @@
 // parts, the first tile, the merge: 11 to 13 thousand cycles however few keys),
 // and at prompts of several hundred tokens the softmax's VALU work beside the
 // MFMAs.  One workgroup per token and q head on the VALU, which this replaced,
-// against this, us a layer: decode at head_dim 80, 32 heads, pos 1499: 133
-// (with its append launch) -> 9.7; 300-token prompt at head_dim 96, 32 q and 8
-// kv heads: 84 -> 16 (8 layers in one launch: 8.1 each).  The same on
-// v_mfma_f32_16x16x4_f32 without parts: 10.8, 27 and 13.4.  Relative error
-// against 64 bits, before -> now: 2.4e-7 -> 2.0e-7 and 1.6e-7 -> 1.3e-7.
+// against this, us a layer of 8 launched one by one, with the appends: decode at
+// head_dim 80, 32 heads, pos 1499: 132 -> 11.4; 300-token prompt at head_dim 96, 32
+// q and 8 kv heads: 78 -> 16.1 (8 layers in one launch: 67 -> 8.2 each).  With plain
+// parts (see split3) 11.0, 16.0 and 8.1; on v_mfma_f32_16x16x4_f32 without parts 1.1,
+// 1.7 and 1.65 times as long.  Relative error against 64 bits, before -> now: 2.4e-7
+// -> 2.0e-7 and 1.6e-7 -> 1.3e-7.
 #include <algorithm>
 #include <type_traits>
 
